@@ -50,7 +50,8 @@ hipError_t launch_bin_scatter(const T* px, const T* py, const T* sx,
     if (once) {
         if ((e = with_cpt(ob.cpt, [&](auto c) -> hipError_t {
                  constexpr int CPT = decltype(c)::value;
-                 DPEP_LAUNCH(ev3, (k_bin_fill_once<T, CPT>), (unsigned)ob.grid, kOnceThreads,
+                 // one workgroup past the cell blocks publishes the plan
+                 DPEP_LAUNCH(ev3, (k_bin_fill_once<T, CPT>), (unsigned)ob.grid + 1u, kOnceThreads,
                              fill_once_lds<T>(b.S), s, px, py, sx, sy, nc, g, b);
                  return hipSuccess;
              })))

@@ -113,7 +113,8 @@ constexpr unsigned kRegionSlack = 16;
 //
 // Records live in kCountSlots regions per strip (workgroup g reserves its
 // runs in region g % kCountSlots of each strip: the reservation atomics are
-// spread over kCountSlots counters per strip).  K3's workgroup 0 publishes
+// spread over kCountSlots counters per strip).  One workgroup of K3 (the
+// first of a counted step, one of its own in the one-pass form) publishes
 // the step's plan: where the regions are (pbase, pcap) and the K4 / G1 work
 // items.  Within a strip the records are numbered region after region,
 // without the unfilled tail of each region ("strip-relative" numbers).  Two

@@ -221,7 +221,7 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
         if (once) {
             with_cpt(ob.cpt, [&](auto c) -> hipError_t {
                 constexpr int CPT = decltype(c)::value;
-                launch((unsigned)ob.grid, kOnceThreads, fill_once_lds<T>(p.S),
+                launch((unsigned)ob.grid + 1u, kOnceThreads, fill_once_lds<T>(p.S),
                        [&] { k_bin_fill_once<T, CPT>(px, py, sx, sy, nc, g, b); });
                 return hipSuccess;
             });
