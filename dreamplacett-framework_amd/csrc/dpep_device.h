@@ -267,7 +267,8 @@ __device__ __forceinline__ void dft16(vec2_t<T>* v)
     for (int n2 = 1; n2 < 4; ++n2)
 #pragma unroll
         for (int k1 = 1; k1 < 4; ++k1)
-            y[n2][k1] = cmul(y[n2][k1], w16<T, INV>(n2 * k1));
+            y[n2][k1] = n2 * k1 == 4 ? cmul_mi<INV>(y[n2][k1])
+                                     : cmul(y[n2][k1], w16<T, INV>(n2 * k1));
 #pragma unroll
     for (int k1 = 0; k1 < 4; ++k1) {
         C a = y[0][k1], b = y[1][k1], c = y[2][k1], d = y[3][k1];

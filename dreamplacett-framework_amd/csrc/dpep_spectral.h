@@ -173,42 +173,38 @@ __device__ __forceinline__ void dct_post(const vec2_t<T>* buf, int s,
     } else {
         const C za = buf[lds_pad(s)];
         const C zb = buf[lds_pad(L - s)];
-        const C v1 = C{(T)0.5 * (za.x + zb.x), (T)0.5 * (za.y - zb.y)};
-        const C v2 = C{(T)0.5 * (za.y + zb.y), (T)-0.5 * (za.x - zb.x)};
-        const C w1 = cmul(pc, v1);
-        const C w2 = cmul(pc, v2);
-        Xk = C{w1.x * scale, w2.x * scale};
-        Xm = C{-w1.y * scale, -w2.y * scale};
+        // the halves of V1, V2 and the scale (a power of two) in the twiddle:
+        // exact, and once per pair instead of once per value
+        const C c = C{pc.x * ((T)0.5 * scale), pc.y * ((T)0.5 * scale)};
+        const C v1 = C{za.x + zb.x, za.y - zb.y};
+        const C v2 = C{za.y + zb.y, zb.x - za.x};
+        Xk = C{c.x * v1.x - c.y * v1.y, c.x * v2.x - c.y * v2.y};
+        Xm = C{-c.y * v1.x - c.x * v1.y, -c.y * v2.x - c.x * v2.y};
     }
 }
 
-// Inverse pre-processing of slot s for one real spectrum given X[k], X[m]
-// (k = s, m = L - s; for s = 0: k = 0, m = L/2).  rev selects X'[k] = X[L-k].
-template <typename T, int L>
-__device__ __forceinline__ void inv_pre(int s, T xk, T xm, bool rev, vec2_t<T> c,
-                                        vec2_t<T>& Vk, vec2_t<T>& Vm)
+// Inverse pre-processing of slot s for two packed spectra (V = V1 + i V2).
+// Each spectrum gives a = X[k], b = X[m] (k = s, m = L - s), or with the
+// reversed spectrum X'[k] = X[L-k] of the S transform a = X[m], b = X[k]:
+//   V[k] = conj(c) (a - i b),  V[m] = i c (b - i a)
+// The two spectra are added before the multiplication by the twiddle, which
+// they share: one complex product per output instead of two (12 operations
+// per pair where forming each V and adding took 24).  Slot 0 owns k = 0,
+// where V[0] = (z1, z2) (X[0], or 0 of a reversed spectrum), and m = L/2,
+// where a = b = X[L/2] = (m1, m2); c = exp(-i pi/4) there, so V[L/2] has the
+// form of V[m].
+template <typename T>
+__device__ __forceinline__ void inv_pre(int s, T a1, T b1, T a2, T b2, vec2_t<T> z,
+                                        vec2_t<T> m, vec2_t<T> c, vec2_t<T>& Vk,
+                                        vec2_t<T>& Vm)
 {
     using C = vec2_t<T>;
-    if (s == 0) {
-        Vk = C{rev ? (T)0 : xk, (T)0};
-        // conj(c) * (xm - i xm)
-        Vm = C{c.x * xm - c.y * xm, -c.x * xm - c.y * xm};
-    } else {
-        const T a = rev ? xm : xk;
-        const T b = rev ? xk : xm;
-        // conj(c) * (a - i b)
-        Vk = C{c.x * a - c.y * b, -c.x * b - c.y * a};
-        // i * c * (b - i a) = i*(c.x b + c.y a) + ... expand:
-        // c*(b - i a) = (c.x b + c.y a) + i (c.y b - c.x a); times i:
-        Vm = C{-(c.y * b - c.x * a), c.x * b + c.y * a};
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ vec2_t<T> pack2(vec2_t<T> v1, vec2_t<T> v2)
-{
-    // v1 + i v2
-    return vec2_t<T>{v1.x - v2.y, v1.y + v2.x};
+    const C p = C{a1 + b2, a2 - b1};
+    C q = C{b1 + a2, b2 - a1};
+    if (s == 0) q = C{m.x + m.y, m.y - m.x};
+    Vk = C{c.x * p.x + c.y * p.y, c.x * p.y - c.y * p.x};
+    Vm = C{-c.x * q.y - c.y * q.x, c.x * q.x - c.y * q.y};
+    if (s == 0) Vk = z;
 }
 
 // ---------------------------------------------------------------------------
@@ -321,11 +317,12 @@ __global__ __launch_bounds__(col_threads<T>(L)) void k_col_pass(
             const T b1m = Am[i].x * w1m;
             const T b2k = Ak[i].y * w2k;
             const T b2m = Am[i].y * w2m;
-            C p1k, p1m, p2k, p2m;
-            inv_pre<T, L>(s, b1k, b1m, rev, pst[i], p1k, p1m);
-            inv_pre<T, L>(s, b2k, b2m, rev, pst[i], p2k, p2m);
-            Vk[i] = pack2<T>(p1k, p2k);
-            Vm[i] = pack2<T>(p1m, p2m);
+            if (rev)
+                inv_pre<T>(s, b1m, b1k, b2m, b2k, C{(T)0, (T)0}, C{b1m, b2m}, pst[i], Vk[i],
+                           Vm[i]);
+            else
+                inv_pre<T>(s, b1k, b1m, b2k, b2m, C{b1k, b2k}, C{b1m, b2m}, pst[i], Vk[i],
+                           Vm[i]);
         }
         __syncthreads();   // previous round's readers of buf are done
 #pragma unroll
@@ -447,11 +444,7 @@ __global__ __launch_bounds__(row_threads<T>(L), row_waves<T>()) void k_row_inv(
             const int s = t + TPF * i;
             const C zk = buf[lds_pad(s)];
             const C zm = buf[lds_pad(s == 0 ? L / 2 : L - s)];
-            C pxk, pxm, pyk, pym;
-            inv_pre<T, L>(s, zk.x, zm.x, false, pst[i], pxk, pxm);
-            inv_pre<T, L>(s, zk.y, zm.y, true, pst[i], pyk, pym);
-            Vk[i] = pack2<T>(pxk, pyk);
-            Vm[i] = pack2<T>(pxm, pym);
+            inv_pre<T>(s, zk.x, zm.x, zm.y, zk.y, C{zk.x, (T)0}, zm, pst[i], Vk[i], Vm[i]);
         }
         __syncthreads();
 #pragma unroll
@@ -512,11 +505,8 @@ __global__ __launch_bounds__(row_threads<T>(L), row_waves<T>()) void k_row_inv(
             const C zm = buf[lds_pad(m)];
             // Up = Uy / w_v at the slot's two columns (column 0: / w_v(1))
             const T rk = fast_rcp((T)(s > 0 ? s : 1) * wv), rm = fast_rcp((T)m * wv);
-            C pak, pam, pbk, pbm;
-            inv_pre<T, L>(s, zk.x * rk, zm.x * rm, false, pst[i], pak, pam);
-            inv_pre<T, L>(s, zk.y * rk, zm.y * rm, false, pst[i], pbk, pbm);
-            Vk[i] = pack2<T>(pak, pbk);
-            Vm[i] = pack2<T>(pam, pbm);
+            const C xk = C{zk.x * rk, zk.y * rk}, xm = C{zm.x * rm, zm.y * rm};
+            inv_pre<T>(s, xk.x, xm.x, xk.y, xm.y, xk, xm, pst[i], Vk[i], Vm[i]);
         }
         __syncthreads();
 #pragma unroll
