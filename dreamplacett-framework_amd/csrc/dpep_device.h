@@ -177,7 +177,7 @@ __host__ __device__ constexpr int lds_len(int L) { return L + (L >> 5) + 8; }
 
 // 16-byte vector of T (global loads and stores of the spectral passes).
 template <typename T, int V = 16 / (int)sizeof(T)>
-struct alignas(16) pack {
+struct alignas(V * sizeof(T)) pack {
     T v[V];
 };
 

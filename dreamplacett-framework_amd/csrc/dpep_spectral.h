@@ -82,10 +82,29 @@ __host__ __device__ constexpr int row_e(int L)
     return small_e<T>(L);
 }
 
+// FFTs of one column-pass workgroup: fpw, or fewer where the tile's columns
+// are split over several workgroups (neighbours on one XCD, which share the
+// tiles' cache lines).  The pass holds ~200 VGPRs (float64 ~430), so a SIMD
+// has two waves (one) and a barrier of a large workgroup leaves it idle;
+// workgroups of their own phases overlap instead.  Measured, us per step with
+// one workgroup per tile -> split: 512^2 40.05 -> 39.7 (one FFT is one wave),
+// float64 52.4 -> 51.8; 1024^2 61.4 -> 60.0 (two FFTs; one: 60.9); 4096^2
+// 411.5 -> 405.8; 2048^2 float64 229.7 -> 227.9.  At 2048 float32 two FFTs
+// stay together (one each: 118.3 -> 120.5), and below 512, where one would
+// leave most of a wave empty (128^2 +0.2).  At 8192 one FFT (512 threads)
+// may hold 256 VGPRs: 28 spilled instead of 165.
 template <typename T>
-__host__ __device__ constexpr int col_threads(int L)
+__host__ __device__ constexpr int col_f(int L)
 {
-    return fpw<T>(L) * (L / col_e<T>(L));
+    const bool two = L < 512 || (sizeof(T) == 4 && (L == 1024 || L == 2048));
+    return two ? 2 : 1;
+}
+
+// Threads of a column-pass workgroup of F FFTs (0: fpw, a whole tile's).
+template <typename T>
+__host__ __device__ constexpr int col_threads(int L, int F = 0)
+{
+    return (F ? F : fpw<T>(L)) * (L / col_e<T>(L));
 }
 
 template <typename T>
@@ -212,14 +231,15 @@ __device__ __forceinline__ void inv_pre(int s, T a1, T b1, T a2, T b2, vec2_t<T>
 // three inverse transforms along x; writes Ux, Uy and Up (Up over T) tiled.
 // ---------------------------------------------------------------------------
 template <typename T, int L, int F, bool kSq>
-__global__ __launch_bounds__(col_threads<T>(L)) void k_col_pass(
+__global__ __launch_bounds__((col_threads<T>(L, F))) void k_col_pass(
     SpectralArgs a, const T* __restrict__ Tt, T* __restrict__ Ux,
     T* __restrict__ Uy)
 {
     constexpr Tiles kT = square_tiles<T, L>();
     using C = vec2_t<T>;
     constexpr int E = col_e<T>(L), TPF = L / E, NT = F * TPF, LP = lds_len(L);
-    constexpr int TV = 2 * F;
+    // a tile's TV columns, CW of them this workgroup's (2 per FFT)
+    constexpr int TV = 2 * fpw<T>(L), CW = 2 * F, SUB = TV / CW;
     extern __shared__ __align__(16) unsigned char smem[];
     C* sb = reinterpret_cast<C*>(smem);
     const int tid = threadIdx.x, f = tid / TPF, t = tid % TPF;
@@ -230,30 +250,29 @@ __global__ __launch_bounds__(col_threads<T>(L)) void k_col_pass(
     const int lgTXT = __builtin_ctz(TXT);
     // tile offsets by shifts: every tile extent and N are powers of two
     const int lgNBV = __builtin_ctz(kSq ? L : a.N) - __builtin_ctz(TV);
-    const int b2 = blockIdx.x;
-    const int v0 = b2 * TV;
-    constexpr int lgTV = __builtin_ctz(TV);
-    const int tile_elems = TX * TV;
+    const int lb = SUB > 1 ? (int)xcd_logical_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+    const int b2 = lb / SUB, sub = lb % SUB;
+    const int v0 = b2 * TV + sub * CW;
+    constexpr int lgTV = __builtin_ctz(TV), lgCW = __builtin_ctz(CW);
     const int lgTE = lgTX + lgTV;
 
     // load the tiles (bx, b2) of T for every bx: each vector holds V
     // consecutive columns v (pairs of them form the complex input of one
     // FFT) of one x
-    constexpr int V = kVec<T>, NV = L * TV / (NT * V);
-    static_assert(NV * NT * V == L * TV && V % 2 == 0 && TV % V == 0, "P2 vector split");
+    constexpr int V = kVec<T> < CW ? kVec<T> : CW, NV = L * CW / (NT * V);
+    static_assert(NV * NT * V == L * CW && V % 2 == 0 && CW % V == 0, "P2 vector split");
     const C* post = reinterpret_cast<const C*>(a.postM);
     C pst[E / 2];           // post-processing twiddles of the thread's slots
     FftTw<T, L, E> twp;     // and its FFT twiddles (forward; inverse conjugates)
     {
-        const int tile_t = TXT * TV;
         const int lgTET = lgTXT + lgTV;
-        pack<T> r[NV];
+        pack<T, V> r[NV];
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int e0 = (tid + i * NT) * V;
-            const int bx = e0 >> lgTET;
-            const int w = e0 & (tile_t - 1);
-            r[i] = *reinterpret_cast<const pack<T>*>(
+            const int x = e0 >> lgCW, bx = x >> lgTXT;
+            const int w = ((x & (TXT - 1)) << lgTV) + sub * CW + (e0 & (CW - 1));
+            r[i] = *reinterpret_cast<const pack<T, V>*>(
                 Tt + (((((unsigned)bx << lgNBV) + (unsigned)b2) << lgTET) + (unsigned)w));
         }
 #pragma unroll
@@ -262,10 +281,7 @@ __global__ __launch_bounds__(col_threads<T>(L)) void k_col_pass(
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int e0 = (tid + i * NT) * V;
-            const int bx = e0 >> lgTET;
-            const int w = e0 & (tile_t - 1);
-            const int x = (bx << lgTXT) + (w >> lgTV);
-            const int v_in = w & (TV - 1);
+            const int x = e0 >> lgCW, v_in = e0 & (CW - 1);
             const int px = lds_pad(makhoul_pos<L>(x));
 #pragma unroll
             for (int q = 0; q < V; q += 2)
@@ -339,20 +355,18 @@ __global__ __launch_bounds__(col_threads<T>(L)) void k_col_pass(
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
             const int e0 = (tid + i * NT) * V;
-            const int bx = e0 >> lgTE;
-            const int w = e0 & (tile_elems - 1);
-            const int x = (bx << lgTX) + (w >> lgTV);
-            const int v_in = w & (TV - 1);
+            const int x = e0 >> lgCW, bx = x >> lgTX, v_in = e0 & (CW - 1);
+            const int w = ((x & (TX - 1)) << lgTV) + sub * CW + v_in;
             const int px = lds_pad(makhoul_pos<L>(x));
             const T sc = (round == 0 && (x & 1)) ? -rscale : rscale;
-            pack<T> o;
+            pack<T, V> o;
 #pragma unroll
             for (int q = 0; q < V; q += 2) {
                 const C z = sb[((v_in + q) >> 1) * LP + px];
                 o.v[q] = z.x * sc;
                 o.v[q + 1] = z.y * sc;
             }
-            *reinterpret_cast<pack<T>*>(
+            *reinterpret_cast<pack<T, V>*>(
                 dst + (((((unsigned)bx << lgNBV) + (unsigned)b2) << lgTE) + (unsigned)w)) = o;
         }
     }

@@ -18,6 +18,12 @@ constexpr size_t lds_bytes()
     return (size_t)fpw<T>(L) * lds_len(L) * sizeof(vec2_t<T>);
 }
 
+template <typename T, int L>
+constexpr size_t col_lds()     // the column pass's
+{
+    return (size_t)col_f<T>(L) * lds_len(L) * sizeof(vec2_t<T>);
+}
+
 template <typename T, typename Fn>
 static hipError_t dispatch_len(int L, Fn&& fn)
 {
@@ -71,13 +77,13 @@ hipError_t launch_col_pass(const SpectralArgs& a, const T* Tt, T* Ux, T* Uy,
 {
     return dispatch_len<T>(a.M, [&](auto lc) -> hipError_t {
         constexpr int L = decltype(lc)::value;
-        constexpr int F = fpw<T>(L);
-        const dim3 grid(a.N / (2 * F)), block(col_threads<T>(L));
+        constexpr int F = col_f<T>(L);
+        const dim3 grid(a.N / (2 * F)), block(col_threads<T>(L, F));
         if (square_form<T, L>(a))
             DPEP_LAUNCH(ev, (k_col_pass<T, L, F, true>), grid, block,
-                        (lds_bytes<T, L>()), s, a, Tt, Ux, Uy);
+                        (col_lds<T, L>()), s, a, Tt, Ux, Uy);
         else
-            DPEP_LAUNCH(ev, (k_col_pass<T, L, F, false>), grid, block, (lds_bytes<T, L>()), s,
+            DPEP_LAUNCH(ev, (k_col_pass<T, L, F, false>), grid, block, (col_lds<T, L>()), s,
                         a, Tt, Ux, Uy);
         return hipGetLastError();
     });
@@ -109,13 +115,13 @@ static hipError_t prepare_len()
     const int bytes = (int)lds_bytes<T, L>();
     hipError_t e;
     constexpr bool kSq = L >= kSquareMin;
-    if ((e = hipFuncSetAttribute((const void*)k_col_pass<T, L, F, false>,
+    if ((e = hipFuncSetAttribute((const void*)k_col_pass<T, L, col_f<T>(L), false>,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes)) ||
         (e = hipFuncSetAttribute((const void*)k_row_inv<T, L, F, false>,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, bytes)))
         return e;
     if constexpr (kSq) {
-        if ((e = hipFuncSetAttribute((const void*)k_col_pass<T, L, F, true>,
+        if ((e = hipFuncSetAttribute((const void*)k_col_pass<T, L, col_f<T>(L), true>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize, bytes)))
             return e;
         return hipFuncSetAttribute((const void*)k_row_inv<T, L, F, true>,

@@ -243,9 +243,9 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
         for (int s2 = 0; s2 < kSideWords * p.S; ++s2)
             if (b.bigflag[s2]) { fprintf(stderr, "bigflag left set\n"); return 4; }
         {
-            constexpr int F = fpw<T>(LM);
+            constexpr int F = col_f<T>(LM);
             const size_t shm = (size_t)F * lds_len(LM) * sizeof(vec2_t<T>);
-            launch(N / (2 * F), col_threads<T>(LM), shm, [&] { col_pass_as_launched<T, LM, F>(a, Tt, Ux, Uy); });
+            launch(N / (2 * F), col_threads<T>(LM, F), shm, [&] { col_pass_as_launched<T, LM, F>(a, Tt, Ux, Uy); });
         }
         {
             constexpr int F = fpw<T>(LN);
@@ -385,9 +385,9 @@ static int run_spectral()
     T* Ux = exact<T>(mn); T* Uy = exact<T>(mn);
     T* fx = exact<T>(mn); T* fy = exact<T>(mn); T* phi = exact<T>(mn);
     {
-        constexpr int F = fpw<T>(LM);
+        constexpr int F = col_f<T>(LM);
         const size_t shm = (size_t)F * lds_len(LM) * sizeof(vec2_t<T>);
-        launch(N / (2 * F), col_threads<T>(LM), shm, [&] { col_pass_as_launched<T, LM, F>(a, Tt, Ux, Uy); });
+        launch(N / (2 * F), col_threads<T>(LM, F), shm, [&] { col_pass_as_launched<T, LM, F>(a, Tt, Ux, Uy); });
     }
     {
         constexpr int F = fpw<T>(LN);
