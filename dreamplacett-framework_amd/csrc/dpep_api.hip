@@ -144,7 +144,7 @@ static void release(dpep_ctx* c)
                     c->d_postM, c->d_twN, c->d_postN, b.cnt, b.xtot, b.pbase,
                     b.pcap, b.pool_n, b.ovst, b.oruns, b.items, b.nitems, b.done, b.recg,
                     b.recm, b.pos, b.gtmp,
-                    b.bigflag, b.B, b.chunk, b.items_g, c->d_raw};
+                    b.bigflag, b.B, b.chunk, b.items_g, b.tall_n, b.tall_cell, c->d_raw};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev)
@@ -177,7 +177,8 @@ static int run_step(dpep_ctx* c, const T* px, const T* py, const T* sx,
         (gather && (!gx || !gy)) || !b.cnt || !b.pbase || !b.pcap ||
         !b.pool_n || !b.ovst || !b.oruns || !b.items || !b.nitems || !b.done || !b.recg ||
         !b.recm || !b.pos ||
-        !b.gtmp || !b.bigflag || !b.B || !b.chunk || !b.items_g)
+        !b.gtmp || !b.bigflag || !b.B || !b.chunk || !b.items_g || !b.tall_n ||
+        !b.tall_cell)
         return fail(DPEP_ERR_STATE, "internal: a kernel argument is NULL");
     if (nc > c->nc_max)
         return fail(DPEP_ERR_ARG, "nc=%d exceeds nc_max=%d", nc, c->nc_max);
@@ -185,6 +186,7 @@ static int run_step(dpep_ctx* c, const T* px, const T* py, const T* sx,
         HIP_TRY(hipMemsetAsync(b.xtot, 0, 2 * (size_t)kCountSlots * b.S * sizeof(unsigned), s));
         HIP_TRY(hipMemsetAsync(b.pool_n, 0, 2 * sizeof(unsigned), s));
         HIP_TRY(hipMemsetAsync(b.ovst, 0, 2 * (size_t)b.S * sizeof(unsigned long long), s));
+        HIP_TRY(hipMemsetAsync(b.tall_n, 0, 2 * (size_t)b.S * sizeof(unsigned), s));
         c->scrub = 0;
     }
     // one pass over the cells when the previous step left its counts
@@ -393,6 +395,11 @@ int dpep_create(int M, int N, int nc_max, double xl, double yl, double xh,
         HIP_TRY(hipMalloc(&b.gtmp, nrec * 2 * c->esz));
         HIP_TRY(hipMalloc((void**)&b.bigflag, (size_t)kSideWords * p.S * sizeof(unsigned)));
         HIP_TRY(hipMalloc(&b.B, (size_t)M * N * accb));
+        // per-strip lists of tall cells
+        b.tall_cap = kTallCap;
+        HIP_TRY(hipMalloc((void**)&b.tall_n, 2 * (size_t)p.S * sizeof(unsigned)));
+        HIP_TRY(hipMemset(b.tall_n, 0, 2 * (size_t)p.S * sizeof(unsigned)));
+        HIP_TRY(hipMalloc(&b.tall_cell, (size_t)p.S * kTallCap * 4 * c->esz));
         // B and the strip flags must start at zero; each step leaves them so.
         HIP_TRY(hipMemset(b.B, 0, (size_t)M * N * accb));
         HIP_TRY(hipMemset(b.bigflag, 0, (size_t)kSideWords * p.S * sizeof(unsigned)));

@@ -21,8 +21,8 @@
 //                 block of cells per workgroup (once_blocks); records
 //                 past a region's room -> overflow pool, with their
 //                 strip (K4 and G1 pick their strip's pool records out
-//                 of it); tall cells added to B by 16-thread teams at
-//                 the block's end
+//                 of it); tall cells entered in their strips' lists
+//                 by 16-thread teams at the block's end
 //   k_strip_acc   one work item = (strip, chunk): LDS accumulate,     K4
 //                 flush rho = D0 + tile (+B); the chunks of a split
 //                 strip add into B and the last one to finish flushes
@@ -53,10 +53,12 @@
 // forces in cell order instead of G1 scattering them.
 //
 // A cell whose span covers more than R rows or more than kMaxSpanY + 1
-// columns ("tall") skips the sort: K3 adds it with global atomics into the
-// side map B (zero between steps) and marks the column blocks it touches in
-// each of its strips; K4 folds and re-zeroes those blocks of B, and G2
-// gathers the cell with a team of threads.  Every other cell touches at most
+// columns ("tall") skips the sort.  The one-pass K3 enters it in the list of
+// every strip it touches and K4 adds its bins in the strip's LDS tile
+// (list_tall_team); a counted K3, and a list that is full, adds it with global
+// atomics into the side map B (zero between steps) and marks the column blocks
+// it touches in each of its strips, and K4 folds and re-zeroes those blocks
+// of B.  G2 gathers the cell with a team of threads.  Every other cell touches at most
 // two strips, so the record arrays hold 2*nc_max.
 #pragma once
 
@@ -1123,17 +1125,49 @@ __device__ __forceinline__ void record_density(const vec4_t<T>& rg, unsigned rm,
 // gather).
 constexpr int kTallTeam = 16;
 
-// A tall cell's density added into the side map B by a team of kTallTeam
-// threads (lane: index in the team; every lane calls it for the same cell,
-// its px, py, sx, sy): its bins strided over the team, each the value
-// a single thread's row-by-row loop adds, (ratio / bin area * tx) * ty in
-// fixed point, so the sums are bitwise the same in any order; the lanes
-// also mark the cell's column blocks in each of its strips.  One thread per
+// A tall cell's density over rows [ka, kb], one value per bin, by a team of
+// kTallTeam threads (lane: index in the team; every lane calls it for the same
+// cell): add(row, column, fixed-point value) for the bins strided over the
+// team.  Each is the value a single thread's row-by-row loop adds, (ratio /
+// bin area * tx) * ty in fixed point, so the sums are bitwise the same in any
+// order and whether B or a strip's LDS tile receives them.  One thread per
 // tall cell held its workgroup ~10 us for a cell of ~50 bins (float64).
+template <typename Fn>
+__device__ __forceinline__ void tall_density(const CellSpan& c, int ka, int kb, int lane,
+                                             const Grid& g, Fn&& add)
+{
+    const double sc = c.ratio() * g.inv_ba;
+    const int ny1 = c.byh - c.byl + 1;
+    const int nb = (kb - ka + 1) * ny1;
+    for (int e = lane; e < nb; e += kTallTeam) {
+        const int k = ka + e / ny1, q = c.byl + e % ny1;
+        const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
+        const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
+        if (tx <= 0.0 || ty <= 0.0) continue;
+        const double stx = sc * tx;
+        add(k, q, to_fixed(stx * ty, g.fix_scale));
+    }
+}
+
+// One tall cell of a one-pass step, by a team of kTallTeam threads: an entry
+// in the list of every strip it touches, from which K4 adds its bins in the
+// strip's LDS tile.  A strip whose list is full takes the cell's bins in its
+// rows through the side map B instead (marked for K4's fold), and so do all
+// strips of a cell of more than kTallStrips strips or kTallBins bins in a
+// strip (a team would walk it for long).  The sums are bitwise the same.
+// Through B, a strip with any tall cell pays a dependent round of loads in K4
+// and a read and a rewrite of the marked blocks of 64-bit words: 12 K tall
+// cells of 2.0 M on 4096 x 4096 (a quarter of B marked) K4 104.7 -> 82.0 us and
+// K3 54.8 -> 52.7, ~300 of 210 K on 2048 x 2048 step 99.2 -> 95.  (Gathering
+// them in G1 the same way, partials per strip summed by G2, made G1 11 us
+// slower at 4096 x 4096 against 2 us won in G2.)
+constexpr int kTallStrips = 32;
+constexpr int kTallBins = 512;
+
 template <typename T>
-__device__ __forceinline__ void scatter_tall_team(const vec4_t<T>& cell, int lane,
-                                                  const Grid& g, const BinArgs& b,
-                                                  unsigned long long* __restrict__ Bm)
+__device__ __forceinline__ void list_tall_team(const vec4_t<T>& cell, int lane,
+                                               const Grid& g, const BinArgs& b,
+                                               unsigned long long* __restrict__ Bm)
 {
     CellSpan c;
     if (!cell_span((double)cell.x, (double)cell.y, (double)cell.z, (double)cell.w, g, c))
@@ -1141,20 +1175,27 @@ __device__ __forceinline__ void scatter_tall_team(const vec4_t<T>& cell, int lan
     int s0, s1;
     bool tall;
     cell_strips<T>(c, g, b.R, b.lgR, s0, s1, tall);
-    const double sc = c.ratio() * g.inv_ba;
-    const int ny1 = c.byh - c.byl + 1;
-    const int nb = (c.bxh - c.bxl + 1) * ny1;
-    for (int e = lane; e < nb; e += kTallTeam) {
-        const int k = c.bxl + e / ny1, q = c.byl + e % ny1;
-        const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
-        const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
-        if (tx <= 0.0 || ty <= 0.0) continue;
-        const double stx = sc * tx;
-        atomicAdd(&Bm[(size_t)k * g.N + q], to_fixed(stx * ty, g.fix_scale));
+    unsigned refused = ~0u;                     // bit j: strip s0 + j
+    if (b.tall_n && s1 - s0 < kTallStrips && b.R * (c.byh - c.byl + 1) <= kTallBins) {
+        refused = 0u;
+        for (int s = s0 + lane; s <= s1; s += kTallTeam) {
+            const unsigned e = atomicAdd(&b.tall_n[(size_t)(b.par & 1) * b.S + s], 1u);
+            if (e < b.tall_cap)
+                reinterpret_cast<vec4_t<T>*>(b.tall_cell)[(size_t)s * b.tall_cap + e] = cell;
+            else
+                refused |= 1u << (s - s0);
+        }
+#pragma unroll
+        for (int m = kTallTeam / 2; m > 0; m >>= 1) refused |= __shfl_xor(refused, m, kTallTeam);
+        if (refused == 0u) return;              // uniform across the team
     }
+    auto through_b = [&](int s) { return s - s0 >= kTallStrips || ((refused >> (s - s0)) & 1u); };
+    tall_density(c, c.bxl, c.bxh, lane, g, [&](int k, int q, unsigned long long v) {
+        if (through_b(k >> b.lgR)) atomicAdd(&Bm[(size_t)k * g.N + q], v);
+    });
     const int CB = side_block(g.N);
     for (int s = s0 + lane; s <= s1; s += kTallTeam)
-        side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
+        if (through_b(s)) side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
 }
 
 // ---------------------------------------------------------------------------
@@ -1173,9 +1214,9 @@ __device__ __forceinline__ void scatter_tall_team(const vec4_t<T>& cell, int lan
 // as an earlier form did, cost 60 us at 1.1M cells when 3.5 % of the
 // records overflowed: those atomics execute beyond the XCD's L2, and the
 // overflow of a changed placement gathers on the strips that grew.)
-// Tall cells are listed as they are found (their index; the coordinates of
-// the first kTallList too) and added into B by teams of threads at the end
-// (scatter_tall_team), where no per-cell registers are live.
+// Tall cells are noted as they are found (their index; the coordinates of
+// the first kTallList too) and entered in their strips' lists by teams of
+// threads at the end (list_tall_team), where no per-cell registers are live.
 // LDS: start[S] | room[S] | cnt[S] (the expected strip totals while the plan
 // is made) | tmp[kOnceThreads + kChunkCands] | pool count, pool base | tall
 // count | tall cells[kOnceThreads * kOnceMaxCpt] | (16-byte aligned) the
@@ -1379,7 +1420,7 @@ __global__ __launch_bounds__(kOnceThreads, (once_waves<T, CPT>())) void k_bin_fi
         const vec4_t<T> cell = t < (unsigned)kTallList
                                    ? tall_cell[t]
                                    : vec4_t<T>{px[i], py[i], sx[i], sy[i]};
-        scatter_tall_team<T>(cell, lane, g, b, Bm);
+        list_tall_team<T>(cell, lane, g, b, Bm);
     }
 }
 
@@ -1538,6 +1579,9 @@ __global__ __launch_bounds__(kAccThreads) void k_strip_acc(
         unsigned long long* ost = overflow_state(b, b.par ^ 1);
         for (int e = tid; e < b.S; e += kAccThreads) ost[e] = 0ull;
         if (tid == 0) b.pool_n[(b.par ^ 1) & 1] = 0u;
+        if (b.tall_n)
+            for (int e = tid; e < b.S; e += kAccThreads)
+                b.tall_n[(size_t)((b.par ^ 1) & 1) * b.S + e] = 0u;
     }
     if (w >= (int)b.nitems[0]) return;          // uniform across the group
     const uint4 item = b.items[w];
@@ -1551,6 +1595,10 @@ __global__ __launch_bounds__(kAccThreads) void k_strip_acc(
     // than two ahead)
     StripMap sm;
     strip_map(b, s, sm);
+    // the strip's listed tall cells, for its first chunk
+    unsigned nt = 0u;
+    if (b.tall_n && (item.x >> 16) == 0u)       // uniform across the group
+        nt = min(b.tall_n[(size_t)(b.par & 1) * b.S + s], b.tall_cap);
     constexpr bool kTwL = acc_twiddles_in_lds<T, L>();
     C* twl = reinterpret_cast<C*>(smem + acc_lds_main<T, L>());   // kTwL: W^m, m < L
     if constexpr (kTwL) {   // read at the row DCT, many barriers on
@@ -1569,7 +1617,24 @@ __global__ __launch_bounds__(kAccThreads) void k_strip_acc(
         rgn = recg[r];
         rmn = rec_m<T>(b, r);
     }
+    const vec4_t<T>* tlist =
+        reinterpret_cast<const vec4_t<T>*>(b.tall_cell) + (size_t)s * b.tall_cap;
+    constexpr unsigned kTeams = kAccThreads / kTallTeam;
+    vec4_t<T> tn{};
+    if ((unsigned)(tid / kTallTeam) < nt) tn = tlist[tid / kTallTeam];
     __syncthreads();
+    // the listed tall cells, a team each, before the records (their first
+    // loads are in flight)
+    for (unsigned e = (unsigned)(tid / kTallTeam); e < nt; e += kTeams) {
+        const vec4_t<T> tc = tn;
+        if (e + kTeams < nt) tn = tlist[e + kTeams];
+        CellSpan c;
+        if (cell_span((double)tc.x, (double)tc.y, (double)tc.z, (double)tc.w, g, c))
+            tall_density(c, max(c.bxl, k0), min(c.bxh, k1), tid % kTallTeam, g,
+                         [&](int k, int q, unsigned long long v) {
+                             atomicAdd(&tile[(k - k0) * N + q], v);
+                         });
+    }
     for (unsigned eb = e0 + tid; eb < e1; eb += kAccThreads) {
         const vec4_t<T> rg = rgn;
         const unsigned rm = rmn;

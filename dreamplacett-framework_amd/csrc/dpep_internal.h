@@ -179,6 +179,13 @@ struct BinArgs {
                             // (zero between steps)
     void* B;                // [M*N] uint64, zero between steps: tall cells and
                             // the chunks of split strips add into it
+    // tall cells of a one-pass step, per strip they touch (null: none, every
+    // tall cell through B, as on a counted step)
+    unsigned* tall_n;       // [2][S] entries of the strip, the step of each parity
+                            // (counts the refused ones too; the older set zero
+                            // again after K4)
+    void* tall_cell;        // [S][tall_cap] vec4 of T: px, py, sx, sy
+    unsigned tall_cap;      // entries per strip (kTallCap)
     void* raw;              // [M*N] of T or null: the scattered cells' density
                             // alone (no initial density), written by K4's flush
 };
@@ -307,6 +314,11 @@ inline int run_capacity(long long nc_max)
     const long long nc = nc_max > 0 ? nc_max : 0;
     return (int)(nc / kOnceMinCells + 2);
 }
+
+// Tall cells a strip's list holds: 2.0 M cells on 4096 x 4096 (0.6 % tall)
+// list ~30 per strip; what finds no room goes through the side map.
+constexpr int kTallCap = 512;
+
 struct OnceBlocks {
     int grid;   // blocks (at least one)
     int q;      // cells per block (the last one may hold fewer)

@@ -85,6 +85,8 @@ static void launch(unsigned grid, unsigned block, size_t shm, const std::functio
     ASAN_UNPOISON_MEMORY_REGION(dpep::smem, sizeof(dpep::smem));
 }
 
+static int emu_tall_cap = -1;   // entries of a tall list (-1: the library's)
+
 template <typename T>
 static T* exact(size_t n) { return (T*)malloc(n * sizeof(T) + (n == 0)); }
 
@@ -205,6 +207,14 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
     b.pos = exact<unsigned long long>(nc > 0 ? nc : 1);
     b.gtmp = exact<vec2_t<T>>(nrec);
     b.bigflag = exact<unsigned>(kSideWords * p.S);
+    // the tall cells' lists ("talloff": none, as the no-alloc entry point;
+    // "tallcap=<n>": n entries per strip)
+    if (emu_tall_cap != 0) {
+        b.tall_cap = emu_tall_cap > 0 ? emu_tall_cap : kTallCap;
+        b.tall_n = exact<unsigned>(2 * (size_t)p.S);
+        memset(b.tall_n, 0, 2 * (size_t)p.S * sizeof(unsigned));
+        b.tall_cell = exact<vec4_t<T>>((size_t)p.S * b.tall_cap);
+    }
     b.raw = exact<T>(mn);        // the scatter density without D0, checked below
     b.B = malloc(mn * 8);
     memset(b.B, 0, mn * 8);
@@ -271,6 +281,8 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
         const unsigned* older = b.xtot + (size_t)(b.par ^ 1) * nslot;
         for (size_t s2 = 0; s2 < nslot; ++s2)
             if (older[s2]) { fprintf(stderr, "previous counts left set\n"); return 4; }
+        for (int s2 = 0; b.tall_n && s2 < p.S; ++s2)
+            if (b.tall_n[(size_t)(b.par ^ 1) * p.S + s2]) { fprintf(stderr, "previous tall lists left set\n"); return 4; }
         if (b.pool_n[b.par ^ 1]) { fprintf(stderr, "previous overflow count left set\n"); return 4; }
         for (int s2 = 0; s2 < p.S; ++s2)
             if (b.ovst[(size_t)(b.par ^ 1) * p.S + s2]) { fprintf(stderr, "previous overflow runs left set\n"); return 4; }
@@ -286,10 +298,17 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
     // and must give bitwise step 2's results
     int rc = step(false);
     if (rc) return rc;
+    const std::vector<T> frho(dens, dens + mn), fgx(gx, gx + nc), fgy(gy, gy + nc);
     if (pool_seen) { fprintf(stderr, "fresh step used the pool\n"); return 4; }
     rc = step(true);
     if (rc) return rc;
     if (pool_seen) { fprintf(stderr, "one-pass step on the same cells overflowed (%u)\n", pool_seen); return 4; }
+    // the counted step's tall cells all went through B
+    if (memcmp(frho.data(), dens, mn * sizeof(T)) || memcmp(fgx.data(), gx, nc * sizeof(T)) ||
+        memcmp(fgy.data(), gy, nc * sizeof(T))) {
+        fprintf(stderr, "one-pass step differs from the counted one\n");
+        return 4;
+    }
     std::vector<T> keep[7];
     T* outs[7] = {dens, fx, fy, gx, gy, (T*)b.raw, phi};
     const size_t lens[7] = {mn, mn, mn, (size_t)nc, (size_t)nc, mn, pot ? mn : 0};
@@ -591,6 +610,8 @@ int main(int argc, char** argv)
         if (!strcmp(argv[i], "stage")) stage = true;
         if (!strcmp(argv[i], "off")) off = true;
         if (!strncmp(argv[i], "ch=", 3)) ch = atoi(argv[i] + 3);
+        if (!strcmp(argv[i], "talloff")) emu_tall_cap = 0;
+        if (!strncmp(argv[i], "tallcap=", 8)) emu_tall_cap = atoi(argv[i] + 8);
     }
     return f64 ? dispatch<double>(M, N, nc, det, pot, ch, tall, stage, off)
                : dispatch<float>(M, N, nc, det, pot, ch, tall, stage, off);

@@ -70,6 +70,20 @@ def test_kernels_in_bounds_and_accurate(emu, case):
     assert "emu " in r.stdout
 
 
+# A one-pass step's tall cells through their strips' lists: full lists (three
+# entries a strip: the rest through the side map, the same cell in some strips
+# listed and in others not), split strips, 4-row strips, and no lists at all.
+# The harness compares every output with the counted step's, whose tall cells
+# all take the side map, bit for bit.
+@pytest.mark.parametrize("case", [
+    "f32 64 64 2000 tall tallcap=3", "f64 64 64 1500 tall tallcap=2",
+    "f32 64 64 2000 ch=64 tall tallcap=3", "f32 16 4096 2000 tall tallcap=5",
+    "f64 32 2048 300 tall tallcap=1", "f32 64 64 2000 tall talloff",
+])
+def test_tall_lists(emu, case):
+    test_kernels_in_bounds_and_accurate(emu, case)
+
+
 # The spectral passes alone at every FFT length from 8 to 8192 on either axis
 # (the column pass at 2048 and 4096 rows holds 210-229 VGPRs' worth of state,
 # 8192 the largest LDS use), against the oracle's FFT solve of the same density.
