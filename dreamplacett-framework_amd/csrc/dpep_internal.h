@@ -113,9 +113,8 @@ constexpr unsigned kRegionSlack = 16;
 //
 // Records live in kCountSlots regions per strip (workgroup g reserves its
 // runs in region g % kCountSlots of each strip: the reservation atomics are
-// spread over kCountSlots counters per strip).  One workgroup of K3 (the
-// first of a counted step, one of its own in the one-pass form) publishes
-// the step's plan: where the regions are (pbase, pcap) and the K4 / G1 work
+// spread over kCountSlots counters per strip).  K3's last workgroup, which
+// holds no cells, publishes the step's plan: where the regions are (pbase, pcap) and the K4 / G1 work
 // items.  Within a strip the records are numbered region after region,
 // without the unfilled tail of each region ("strip-relative" numbers).  Two
 // ways to fill:
@@ -238,7 +237,8 @@ inline size_t region_capacity(size_t cap, int S)
 }
 
 // Rows of BinArgs::cnt: an upper bound of the counting workgroups
-// (set_count_blocks) of any step of at most nc cells.  With q >= 1024 cells
+// (set_count_blocks) of any step of at most nc cells, and one more (K3's
+// planning workgroup reads a row, which it does not use).  With q >= 1024 cells
 // per one-pass block and at most kOnceThreads * kOnceMaxCpt, blocks * parts
 // <= (nc / q + 1) * (q / 1024 + 1) <= 2 * nc / 1024 + 3.5.
 inline int count_grid_max(long long nc)

@@ -1,6 +1,7 @@
 // dpep_spectral.hip -- host launchers of the spectral passes (kernels in
 // dpep_spectral.h).
 #include "dpep_spectral.h"
+#include "dpep_tables.h"
 
 namespace dpep {
 
@@ -49,18 +50,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_tables(int L, T* __restrict__ tw,
                                                 T* __restrict__ post)
 {
-    const int i = (int)(blockIdx.x * 256 + threadIdx.x);
-    double s, c;
-    if (i < L) {
-        sincospi(2.0 * (double)i / (double)L, &s, &c);
-        tw[2 * i] = (T)c;
-        tw[2 * i + 1] = (T)-s;
-    }
-    if (i <= L / 2) {
-        sincospi((double)i / (2.0 * (double)L), &s, &c);
-        post[2 * i] = (T)c;
-        post[2 * i + 1] = (T)-s;
-    }
+    table_entry<T>(L, (int)(blockIdx.x * 256 + threadIdx.x), tw, post);
 }
 
 template <typename T>

@@ -238,10 +238,10 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
         } else {
             launch(b.G1, kBinThreads, hist, [&] { k_bin_count<T>(px, py, sx, sy, nc, g, b); });
             if (stage)
-                launch(b.G1, kBinThreads, fill_lds_staged<T>(p.S),
+                launch(b.G1 + 1, kBinThreads, fill_lds_staged<T>(p.S),
                        [&] { k_bin_fill_staged<T>(px, py, sx, sy, nc, g, b); });
             else
-                launch(b.G1, kBinThreads,
+                launch(b.G1 + 1, kBinThreads,
                        (size_t)(2 * p.S + kBinThreads + kChunkCands) * sizeof(unsigned),
                        [&] { k_bin_fill_direct<T>(px, py, sx, sy, nc, g, b); });
         }

@@ -101,3 +101,36 @@ def test_noalloc_limits_and_zero_initial_density(oracle):
         # ... unless the flags drop it (NO_GATHER = 8)
         assert _noalloc(lib, w, np.float32, w.nc, None, cells, w.nc, o2, flags=8) == 0
         db.sync()
+
+
+@pytest.mark.parametrize("M,N", [(256, 1024), (1024, 64), (8, 8)])
+def test_noalloc_tables_of_both_axes(M, N):
+    """Grids whose axes differ in length (two twiddle tables built by the
+    opening kernel; a square grid shares one) and the smallest one: bitwise
+    step_device's outputs."""
+    import dpep
+    lib = dpep.load_library()
+    rng = np.random.default_rng(M * 10007 + N)
+    n = 3001
+
+    class W:
+        xl, yl, xh, yh = 0.0, 0.0, 4000.0, 3000.0
+    W.M, W.N = M, N
+    px, py = rng.uniform(0, 3900, n), rng.uniform(0, 2900, n)
+    sx, sy = rng.uniform(4, 40, n), np.full(n, 12.0)
+    mn = M * N
+    print(f"noalloc tables {M}x{N}", flush=True)
+    with DeviceBuffers() as db:
+        cells = [db.upload(a.astype(np.float32)) for a in (px, py, sx, sy)]
+        oa, ob = ({k: db.alloc((n if k.startswith("grad") else mn) * 4) for k in OUTS}
+                  for _ in range(2))
+        with dpep.Context(M, N, n, W.xl, W.yl, W.xh, W.yh) as ctx:
+            assert lib.dpep_step_device(ctx.handle, *cells, n, *(oa[k] for k in OUTS),
+                                        None) == 0, dpep.last_error()
+            ctx.sync()
+            assert _noalloc(lib, W, np.float32, n, None, cells, n, ob) == 0, dpep.last_error()
+            db.sync()
+            for k in OUTS:
+                m = n if k.startswith("grad") else mn
+                assert np.array_equal(db.download(oa[k], m, np.float32),
+                                      db.download(ob[k], m, np.float32)), k
