@@ -10,10 +10,13 @@
 //   k_row_inv   P3  -> field_x, field_y, potential
 //   k_gather_bin, k_gather_out   per-cell forces <- fields
 #include <math.h>
+#include <signal.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+#include <memory>
 #include <new>
 
 #include <mutex>
@@ -21,6 +24,7 @@
 #include <vector>
 
 #include "dpep.h"
+#include "dpep_copy_pool.h"
 #include "dpep_internal.h"
 
 using namespace dpep;
@@ -56,6 +60,18 @@ constexpr int kNumStages = 7;
 // the context's output buffers, for the validity mask
 constexpr unsigned kOutDensity = 1u, kOutPotential = 2u, kOutFx = 4u, kOutFy = 8u,
                    kOutGx = 16u, kOutGy = 32u, kOutRaw = 64u;
+
+// dpep_step_staged's transfers.  A piece of the link costs ~8 us beside its
+// bytes (57 GB/s), so pieces are large; only the first of an upload and the
+// last of a read-back, whose host copies nothing covers, are short.  One
+// thread copies data the link has just written at ~32 GB/s, three together at
+// more than the link's rate.  1.1M cells, positions in and forces out (host
+// arrays, 1 MiB edge): 922 us as three calls; 890 with no copy thread, 840
+// with one, 639 with two, 651 with three, 655 with five; two with an edge of
+// 512 KiB 740, three with 256 KiB 675, 512 KiB 668, 2 MiB 645.
+constexpr int kStageDepth = 4;
+constexpr size_t kStagePiece = size_t(8) << 20, kStageEdge = size_t(1) << 20;
+constexpr unsigned kStageThreads = 2;
 
 bool is_pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
 
@@ -105,6 +121,10 @@ struct dpep_ctx {
     // and new cells uploaded after the step make every output stale
     unsigned valid = 0;
     float h2d_ms = 0.f, d2h_den_ms = 0.f, d2h_out_ms = 0.f;
+    // dpep_step_staged: the read-back's begin, end of the density and end, the
+    // pieces in flight, and the copy threads (made by the first large copy)
+    hipEvent_t ev_d[3] = {}, ev_p[kStageDepth] = {};
+    std::unique_ptr<CopyPool> copies;
 };
 
 // ---------------------------------------------------------------------------
@@ -154,6 +174,10 @@ static void release(dpep_ctx* c)
     c->prof_ev.clear();
     if (c->ev_x0) (void)hipEventDestroy(c->ev_x0);
     if (c->ev_x1) (void)hipEventDestroy(c->ev_x1);
+    for (auto& e : c->ev_d)
+        if (e) (void)hipEventDestroy(e);
+    for (auto& e : c->ev_p)
+        if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
 }
 
@@ -483,19 +507,27 @@ int dpep_set_fixed_cells(dpep_ctx* c, const void* px, const void* py,
     return rc;
 }
 
-int dpep_set_cells(dpep_ctx* c, const void* px, const void* py,
-                   const void* sx, const void* sy, int nc)
+static int check_cells(const dpep_ctx* c, const void* px, const void* py, const void* sx,
+                       const void* sy, int nc)
 {
-    if (int rc = check_ctx(c)) return rc;
     if (nc < 0 || nc > c->nc_max)
         return fail(DPEP_ERR_ARG, "nc=%d outside [0, nc_max=%d]", nc, c->nc_max);
-    const bool keep_sizes = !sx && !sy;      // positions only
+    const bool keep_sizes = !sx && !sy;
     if (nc > 0 && (!px || !py || (!keep_sizes && (!sx || !sy))))
         return fail(DPEP_ERR_ARG, "cell array is NULL");
     if (keep_sizes && nc > c->nc_sizes)
         return fail(DPEP_ERR_STATE,
                     "sizes kept (sx, sy NULL) for nc=%d cells, but only %d have resident sizes",
                     nc, c->nc_sizes);
+    return DPEP_OK;
+}
+
+int dpep_set_cells(dpep_ctx* c, const void* px, const void* py,
+                   const void* sx, const void* sy, int nc)
+{
+    if (int rc = check_ctx(c)) return rc;
+    const bool keep_sizes = !sx && !sy;      // positions only
+    if (int rc = check_cells(c, px, py, sx, sy, nc)) return rc;
     const size_t bytes = (size_t)nc * c->esz;
     HIP_TRY(hipEventRecord(c->ev_x0, c->stream));
     if (nc > 0) {
@@ -532,15 +564,22 @@ int dpep_sync(dpep_ctx* c)
     return DPEP_OK;
 }
 
+// The outputs a caller asks for are among those the context computes.
+static int check_outputs(const dpep_ctx* c, bool potential, bool grads)
+{
+    if (potential && !c->d_potential)
+        return fail(DPEP_ERR_STATE, "context was created with DPEP_FLAG_NO_POTENTIAL");
+    if (grads && (c->flags & DPEP_FLAG_NO_GATHER))
+        return fail(DPEP_ERR_STATE, "context was created with DPEP_FLAG_NO_GATHER");
+    return DPEP_OK;
+}
+
 int dpep_get_outputs(dpep_ctx* c, void* density, void* potential,
                      void* field_x, void* field_y, void* grad_x, void* grad_y)
 {
     if (int rc = check_ctx(c)) return rc;
     if (!c->stepped) return fail(DPEP_ERR_STATE, "no step has been computed");
-    if (potential && !c->d_potential)
-        return fail(DPEP_ERR_STATE, "context was created with DPEP_FLAG_NO_POTENTIAL");
-    if ((grad_x || grad_y) && (c->flags & DPEP_FLAG_NO_GATHER))
-        return fail(DPEP_ERR_STATE, "context was created with DPEP_FLAG_NO_GATHER");
+    if (int rc = check_outputs(c, potential, grad_x || grad_y)) return rc;
     {
         const unsigned want = (density ? kOutDensity : 0u) | (potential ? kOutPotential : 0u) |
                               (field_x ? kOutFx : 0u) | (field_y ? kOutFy : 0u) |
@@ -614,6 +653,191 @@ int dpep_step(dpep_ctx* c, const void* px, const void* py, const void* sx,
     if ((rc = dpep_compute(c))) return rc;
     return dpep_get_outputs(c, density, potential, field_x, field_y, grad_x,
                             grad_y);
+}
+
+}  // extern "C"
+
+namespace {
+
+// One transfer of dpep_step_staged: device memory, the page-locked buffer it
+// goes through, and the caller's array on the other side (null: none, the
+// staging buffer is the caller's).
+struct Staged {
+    char* dev;
+    char* stage;
+    char* user;
+    size_t bytes;
+};
+
+// A host copy between a caller's array and its staging buffer, on the calling
+// thread and the context's copy threads.  They take pieces of 256 KiB and
+// sleep between copies; a copy of less than two pieces stays on the caller.
+void stage_copy(dpep_ctx* c, void* dst, const void* src, size_t bytes)
+{
+    constexpr size_t kPiece = size_t(256) << 10;
+    if (bytes < 2 * kPiece) {
+        memcpy(dst, src, bytes);
+        return;
+    }
+    if (!c->copies) {
+        const unsigned hw = std::thread::hardware_concurrency();
+        // the threads take no signals: those are the program's own
+        sigset_t all, old;
+        sigfillset(&all);
+        pthread_sigmask(SIG_SETMASK, &all, &old);
+        try {
+            c->copies.reset(new CopyPool((int)std::min(kStageThreads, hw > 1 ? hw - 1 : 0u),
+                                         kPiece));
+        } catch (const std::exception&) {
+        }
+        pthread_sigmask(SIG_SETMASK, &old, nullptr);
+    }
+    if (c->copies)
+        c->copies->copy({{dst, src, bytes}});
+    else
+        memcpy(dst, src, bytes);
+}
+
+// Uploads the arrays, in pieces: while the link moves one piece the host
+// copies the next.  Only the first piece's copy precedes the link, so the
+// first array begins with a short one.  Asynchronous on the context's stream.
+int staged_upload(dpep_ctx* c, const Staged* a, int n)
+{
+    bool first = true;
+    for (int i = 0; i < n; ++i)
+        for (size_t o = 0; o < a[i].bytes;) {
+            size_t len = a[i].bytes - o;
+            if (a[i].user) {
+                len = std::min(len, first && len >= 2 * kStageEdge ? kStageEdge : kStagePiece);
+                stage_copy(c, a[i].stage + o, a[i].user + o, len);
+            }
+            HIP_TRY(hipMemcpyAsync(a[i].dev + o, a[i].stage + o, len, hipMemcpyHostToDevice,
+                                   c->stream));
+            first = false;
+            o += len;
+        }
+    return DPEP_OK;
+}
+
+// Reads the arrays back, in pieces: while the link moves one piece the host
+// copies the one before to the caller's array, at most kStageDepth in flight.
+// Only the last piece's copy follows the link, so the last array ends with a
+// short one.  dens_end: pieces of array 0 .. dens - 1 are followed by that
+// event.  Returns when everything has arrived.
+int staged_readback(dpep_ctx* c, const Staged* a, int n, int dens, hipEvent_t dens_end)
+{
+    struct Piece {
+        char *stage, *user;
+        size_t bytes;
+    } fly[kStageDepth];
+    unsigned issued = 0, taken = 0;
+    auto take = [&]() -> int {
+        const Piece& p = fly[taken % kStageDepth];
+        HIP_TRY(hipEventSynchronize(c->ev_p[taken % kStageDepth]));
+        ++taken;
+        if (p.user) stage_copy(c, p.user, p.stage, p.bytes);
+        return DPEP_OK;
+    };
+    for (int i = 0; i < n; ++i) {
+        for (size_t o = 0; o < a[i].bytes;) {
+            size_t len = a[i].bytes - o;
+            if (a[i].user) {
+                if (len > kStagePiece)
+                    len = kStagePiece;
+                else if (i == n - 1 && len >= 2 * kStageEdge)
+                    len -= kStageEdge;
+            }
+            if (issued - taken == kStageDepth)
+                if (int rc = take()) return rc;
+            const unsigned k = issued % kStageDepth;
+            HIP_TRY(hipMemcpyAsync(a[i].stage + o, a[i].dev + o, len, hipMemcpyDeviceToHost,
+                                   c->stream));
+            HIP_TRY(hipEventRecord(c->ev_p[k], c->stream));
+            fly[k] = {a[i].stage + o, a[i].user ? a[i].user + o : nullptr, len};
+            ++issued;
+            o += len;
+        }
+        if (i == dens - 1) HIP_TRY(hipEventRecord(dens_end, c->stream));
+    }
+    while (taken != issued)
+        if (int rc = take()) return rc;
+    return DPEP_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int dpep_step_staged(dpep_ctx* c, const void* const cells[4], void* const cell_stage[4],
+                     int nc, void* const outputs[6], void* const output_stage[6])
+{
+    if (int rc = check_ctx(c)) return rc;
+    if (!cells || !cell_stage || !outputs || !output_stage)
+        return fail(DPEP_ERR_ARG, "an array of pointers is NULL");
+    if (int rc = check_cells(c, cells[0], cells[1], cells[2], cells[3], nc)) return rc;
+    const bool keep_sizes = !cells[2];
+    const int nin = nc == 0 ? 0 : keep_sizes ? 2 : 4;
+    for (int i = 0; i < nin; ++i)
+        if (!cell_stage[i]) return fail(DPEP_ERR_ARG, "cell staging buffer is NULL");
+    if (int rc = check_outputs(c, output_stage[3], output_stage[4] || output_stage[5]))
+        return rc;
+
+    const size_t mnb = (size_t)c->M * c->N * c->esz, ncb = (size_t)nc * c->esz;
+    Staged in[4], out[6];
+    void* const dev_in[4] = {c->d_px, c->d_py, c->d_sx, c->d_sy};
+    for (int i = 0; i < nin; ++i)
+        in[i] = {(char*)dev_in[i], (char*)cell_stage[i],
+                 cells[i] == cell_stage[i] ? nullptr : (char*)cells[i], ncb};
+    // the density first, as dpep_get_outputs; it has a time of its own
+    void* const dev_out[6] = {c->d_fx, c->d_fy, c->d_density, c->d_potential, c->d_gx, c->d_gy};
+    const int order[6] = {2, 3, 0, 1, 4, 5};
+    int nout = 0;
+    for (int k : order) {
+        const size_t b = k < 4 ? mnb : ncb;
+        if (output_stage[k] && b > 0)
+            out[nout++] = {(char*)dev_out[k], (char*)output_stage[k],
+                           outputs[k] == output_stage[k] ? nullptr : (char*)outputs[k], b};
+    }
+    const int dens = output_stage[2] ? 1 : 0;
+
+    auto run = [&]() -> int {
+        for (auto& e : c->ev_d)
+            if (!e) HIP_TRY(hipEventCreate(&e));
+        for (auto& e : c->ev_p)
+            if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIP_TRY(hipEventRecord(c->ev_x0, c->stream));
+        if (int rc = staged_upload(c, in, nin)) return rc;
+        HIP_TRY(hipEventRecord(c->ev_x1, c->stream));
+        c->nc = nc;
+        c->valid = 0u;
+        if (int rc = dpep_compute(c)) return rc;
+        HIP_TRY(hipEventRecord(c->ev_d[0], c->stream));
+        if (!dens) HIP_TRY(hipEventRecord(c->ev_d[1], c->stream));
+        if (int rc = staged_readback(c, out, nout, dens, c->ev_d[1])) return rc;
+        HIP_TRY(hipEventRecord(c->ev_d[2], c->stream));
+        HIP_TRY(hipEventSynchronize(c->ev_d[2]));
+        return DPEP_OK;
+    };
+    int rc;
+    try {
+        rc = run();
+    } catch (const std::exception& e) {          // std::bad_alloc in a copy's piece list
+        rc = fail(DPEP_ERR_NOMEM, "host copy failed: %s", e.what());
+    }
+    if (rc) {
+        // the staging buffers are the caller's again; which cells are
+        // resident is not known
+        (void)hipStreamSynchronize(c->stream);
+        c->nc = -1;
+        if (!keep_sizes) c->nc_sizes = 0;
+        c->valid = 0u;
+        return rc;
+    }
+    if (!keep_sizes) c->nc_sizes = nc;
+    c->h2d_ms = elapsed(c->ev_x0, c->ev_x1);
+    c->d2h_den_ms = elapsed(c->ev_d[0], c->ev_d[1]);
+    c->d2h_out_ms = elapsed(c->ev_d[1], c->ev_d[2]);
+    return DPEP_OK;
 }
 
 int dpep_step_device(dpep_ctx* c, const void* d_px, const void* d_py,

@@ -1,6 +1,7 @@
-// dpep_copy_pool.h -- the shm server's host copy pool: a fixed set of worker
-// threads that copy lists of (dst, src, bytes) jobs between the shared-memory
-// file and the page-locked staging buffers, with the calling thread taking
+// dpep_copy_pool.h -- the host copy pool of the shm server and of a context's
+// staged step: a fixed set of worker threads that copy lists of (dst, src,
+// bytes) jobs between pageable memory (the shared-memory file, a caller's
+// arrays) and the page-locked staging buffers, with the calling thread taking
 // part.  One memcpy thread moves ~10 GB/s, below the host link, so the
 // server's uploads and read-backs are split over several.
 //
@@ -33,6 +34,7 @@
 #include <algorithm>
 #include <atomic>
 #include <condition_variable>
+#include <exception>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -56,7 +58,12 @@ class CopyPool {
                       Hook hook = nullptr)
         : piece_(piece_bytes ? piece_bytes : 1), hook_(hook)
     {
-        for (int i = 0; i < workers; ++i) threads_.emplace_back([this] { run(); });
+        // a thread the system refuses is done without: the caller takes part
+        threads_.reserve((size_t)(workers > 0 ? workers : 0));
+        try {
+            for (int i = 0; i < workers; ++i) threads_.emplace_back([this] { run(); });
+        } catch (const std::exception&) {
+        }
     }
     ~CopyPool()
     {

@@ -184,6 +184,21 @@ int dpep_step(dpep_ctx* ctx, const void* px, const void* py, const void* sx,
               const void* sy, int nc, void* field_x, void* field_y,
               void* density, void* potential, void* grad_x, void* grad_y);
 
+/* dpep_step with the caller's pageable arrays taken through page-locked
+ * staging buffers (dpep_host_alloc) in pieces: the host copies one piece
+ * while the link moves another, upload, step and read-back follow one another
+ * on the context's stream, and the host waits once at the end.  cells: px,
+ * py, sx, sy (sx and sy both NULL keep the resident sizes); cell_stage: their
+ * staging buffers, nc elements each; cells[i] == cell_stage[i] is already
+ * staged.  output_stage: field_x, field_y, density, potential, grad_x, grad_y
+ * (NULL: not wanted); outputs[i] the caller's array, or NULL or the staging
+ * buffer itself to leave that output there.  A caller's array overlaps no
+ * staging buffer, unless it is its own.  The copies run on the calling thread
+ * and on a few threads of the context.  After an error of the GPU or of host
+ * memory no cells are resident (dpep_set_cells before dpep_compute). */
+int dpep_step_staged(dpep_ctx* ctx, const void* const cells[4], void* const cell_stage[4],
+                     int nc, void* const outputs[6], void* const output_stage[6]);
+
 /* One step on caller-owned device memory, asynchronous on `stream`
  * (a hipStream_t; NULL = the context's stream).  Inputs px..sy hold nc
  * cells.  Outputs may be NULL, in which case they land in the context's own
