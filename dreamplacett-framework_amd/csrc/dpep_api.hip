@@ -56,6 +56,9 @@ int fail(int code, const char* fmt, ...)
 // strip count (+ table), strip fill, strip accumulate (+ row DCT), column
 // pass, row inverse, gather
 constexpr int kNumStages = 7;
+// profile mask of a step whose two gather stages are one kernel: the first
+// of the two, and bit 7
+constexpr unsigned kProfDirect = 0xA0u;
 
 // the context's output buffers, for the validity mask
 constexpr unsigned kOutDensity = 1u, kOutPotential = 2u, kOutFx = 4u, kOutFy = 8u,
@@ -224,13 +227,16 @@ static int run_step(dpep_ctx* c, const T* px, const T* py, const T* sx,
     const size_t slot = prof ? (size_t)(c->prof_steps % c->prof_slots) : 0;
     const hipEvent_t* pe = prof ? &c->prof_ev[slot * 2 * kNumStages] : nullptr;
     if (prof)
-        c->prof_mask[slot] = (unsigned char)((once ? 0u : 1u) | 0x1Eu |
-                                             (gather && nc > 0 ? 0x60u : 0u));
+        c->prof_mask[slot] = (unsigned char)(
+            (once ? 0u : 1u) | 0x1Eu |
+            (!gather || nc <= 0 ? 0u : gather_direct(c->grid, nc, c->esz) ? kProfDirect : 0x60u));
     // a recorded event costs GPU time (a few us per step on MI355X): only
     // when the caller asked for per-step timings
     const bool timed = (c->flags & DPEP_FLAG_STEP_TIMINGS) != 0;
     if (timed) HIP_TRY(hipEventRecord(c->ev[0], s));
-    HIP_TRY(launch_bin_scatter<T>(px, py, sx, sy, nc, c->grid, c->bins, c->sargs, d0n,
+    BinArgs bs = c->bins;
+    if (!gather || gather_direct(c->grid, nc, c->esz)) bs.pos = nullptr;   // G2 alone reads it
+    HIP_TRY(launch_bin_scatter<T>(px, py, sx, sy, nc, c->grid, bs, c->sargs, d0n,
                                   dens, (T*)c->d_T, once, s, pe));
 
     HIP_TRY(launch_col_pass<T>(c->sargs, (T*)c->d_T, (T*)c->d_Ux, (T*)c->d_Uy, s,
@@ -875,7 +881,8 @@ int dpep_get_timings(dpep_ctx* c, float* out)
         // binning (from K1, or K3 on a one-pass step), accumulation and P1
         out[1] = elapsed(pe[(mask & 1u) ? 0 : 2], pe[5]);
         out[5] = elapsed(pe[6], pe[9]);              // P2 + P3
-        out[2] = (mask & 0x60u) ? elapsed(pe[10], pe[13]) : 0.f;   // gather
+        out[2] = (mask & 0x60u)                               // gather
+                     ? elapsed(pe[10], pe[(mask & kProfDirect) == kProfDirect ? 11 : 13]) : 0.f;
     } else {
         out[5] = total;
     }
@@ -937,6 +944,11 @@ int dpep_get_kernel_times(dpep_ctx* c, float* out, int n)
             if (first < 0) first = i;
             last = i;
             if (i < n) out[i] += 1000.f * elapsed(pe[2 * i], pe[2 * i + 1]);
+        }
+        if ((mask & kProfDirect) == kProfDirect) {   // one kernel: half to each stage
+            const float half = 500.f * elapsed(pe[10], pe[11]);
+            if (n > 5) out[5] -= half;
+            if (n > 6) out[6] += half;
         }
         if (n > kNumStages && first >= 0)
             out[kNumStages] += 1000.f * elapsed(pe[2 * first], pe[2 * last + 1]);

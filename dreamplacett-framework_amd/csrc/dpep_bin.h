@@ -280,6 +280,11 @@ __device__ __forceinline__ unsigned long long pos_pair(unsigned p0, unsigned p1)
     return (unsigned long long)p0 | ((unsigned long long)p1 << 32);
 }
 
+__device__ __forceinline__ void put_pos(const BinArgs& b, int i, unsigned long long v)
+{
+    if (b.pos) b.pos[i] = v;        // null (uniform): this step gathers no records
+}
+
 // Strips [s0, s1] a cell occupies and whether it takes the tall path: more
 // rows than a strip, more than kMaxSpanY + 1 columns, or (float32 records,
 // which hold non-negative offsets only) a stretched corner below the die's
@@ -853,7 +858,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_fill_direct(
         if (i >= cend) break;
         CellSpan c;
         if (!cell_span((double)cx[j], (double)cy[j], (double)cw[j], (double)chh[j], g, c)) {
-            b.pos[i] = pos_pair(kPosNone, kPosNone);
+            put_pos(b, i, pos_pair(kPosNone, kPosNone));
             continue;
         }
         int s0, s1;
@@ -876,7 +881,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_fill_direct(
             const int CB = side_block(g.N);
             for (int s = s0; s <= s1; ++s)
                 side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
-            b.pos[i] = pos_pair(kPosTall, kPosNone);
+            put_pos(b, i, pos_pair(kPosTall, kPosNone));
             continue;
         }
         // strip-relative record, evaluated in float64 and rounded once
@@ -892,7 +897,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_fill_direct(
             p1 = atomicAdd(&cur[s1], 1u);
             rec_put<T>(b, recg, p1, geo, rec_span<T>(c.bxl - (s1 << b.lgR), nx, ny, c.byl, true));
         }
-        b.pos[i] = pos_pair(p0, p1);
+        put_pos(b, i, pos_pair(p0, p1));
     }
 }
 
@@ -971,7 +976,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
         if (i >= cend) continue;
         CellSpan c;
         if (!cell_span((double)cx[j], (double)cy[j], (double)cw[j], (double)chh[j], g, c)) {
-            b.pos[i] = pos_pair(kPosNone, kPosNone);
+            put_pos(b, i, pos_pair(kPosNone, kPosNone));
             continue;
         }
         int s0, s1;
@@ -994,7 +999,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
             const int CB = side_block(g.N);
             for (int s = s0; s <= s1; ++s)
                 side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
-            b.pos[i] = pos_pair(kPosTall, kPosNone);
+            put_pos(b, i, pos_pair(kPosTall, kPosNone));
             continue;
         }
         // strip-relative record, evaluated in float64 and rounded once
@@ -1050,7 +1055,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
                 rec_put<T>(b, recg, d1, geo[j], m1[j]);
             }
         }
-        b.pos[i] = pos_pair(d0, d1);
+        put_pos(b, i, pos_pair(d0, d1));
     }
     __syncthreads();
     // staged records out, consecutive threads on consecutive slots: slot k
@@ -1410,7 +1415,7 @@ __global__ __launch_bounds__(kOnceThreads, (once_waves<T, CPT>())) void k_bin_fi
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
         const int i = c0 + tid + j * NT;
-        if (i < cend) b.pos[i] = pos_pair(p0[j], p1[j]);
+        if (i < cend) put_pos(b, i, pos_pair(p0[j], p1[j]));
     }
     // the tall cells, by teams of threads, last: the per-cell arrays above
     // are dead here (earlier, their registers spilled); coordinates past the
@@ -2206,6 +2211,137 @@ __global__ __launch_bounds__(NT) void k_gather_out(
     for (unsigned t = 0; t < n; ++t)          // uniform across the group
         if ((large[t >> 5] >> (t & 31u)) & 1u)
             gather_tall<T, NT>((int)list[t], px, py, sx, sy, g, fx, fy, red, gx, gy);
+}
+
+// ---------------------------------------------------------------------------
+// G1 and G2 in one kernel, for few cells on small maps (gather_direct): a
+// thread per cell evaluates the cell's span again (float64, the record K3
+// would store, so the same offsets and weights) and reads the field bins
+// themselves: 4 columns of a row and field in one 16-byte load, the first
+// kDirRows rows at once, a row the cell does not reach by no lane (the third
+// row of a cell of two loaded all the same measured 0.6-1 us more).  No rows
+// to stage, no partials to write and read back, no heaviest strip, one launch
+// fewer.  Bound by latency (cells, then fields) while the cells are few, then
+// by the L2's lines: ~7 lines of 128 bytes per cell for ~30 used.  Tall cells
+// as in k_gather_out, and cells of more than kDirCols columns with them.
+// Step, us: 5K cells on 128 x 128 30.1 -> 27.0, 150K on 512 x 512 (no-alloc)
+// 46.6 -> 45.1.
+// LDS: gather_out_lds<kDirThreads, 1>.
+// ---------------------------------------------------------------------------
+constexpr int kDirThreads = 256;
+constexpr int kDirRows = 3;
+constexpr int kDirCols = 16;
+
+// 4 field values of a row, aligned to one
+template <typename T>
+struct alignas(sizeof(T)) quad {
+    T v[4];
+};
+
+template <typename T>
+__device__ __forceinline__ vec2_t<T> cell_force(const CellSpan& c, const Grid& g,
+                                                const T* __restrict__ fx,
+                                                const T* __restrict__ fy)
+{
+    const int N = g.N;
+    const double ex = (c.x - (g.xl + c.bxl * g.bsx)) * g.inv_bsx;
+    const double ey = (c.y - (g.yl + c.byl * g.bsy)) * g.inv_bsy;
+    const vec4_t<T> geo = rec_geo<T>(ex, ey, c.sx * g.inv_bsx, c.sy * g.inv_bsy, c.byl, 0);
+    const RecView<T> rv = rec_view<T>(
+        geo, rec_span<T>(0, c.bxh - c.bxl, c.byh - c.byl, c.byl, false), c.bxl, g.stretch, N);
+    const int ka = max(rv.bxl, 0), kb = min(rv.bxl + rv.nx, g.M - 1);
+    // the y overlaps of 4 columns from cb on, zero where not positive; the
+    // 4 lie within the row (N >= 8): where the cell begins past N - 4 the
+    // first ones are not the cell's
+    const int cb = min(rv.byl, N - 4), o = cb - rv.byl;
+    const T yrc = min(rv.yr, (T)(N - rv.byl));
+    T tyv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        tyv[q] = max(min(yrc, (T)(o + q + 1)) - max(rv.dy, (T)(o + q)), (T)0);
+    T ax = (T)0, ay = (T)0;
+    for (int k0 = ka; k0 <= kb; k0 += kDirRows) {
+        quad<T> vx[kDirRows], vy[kDirRows];
+#pragma unroll
+        for (int r = 0; r < kDirRows; ++r) {
+            vx[r] = vy[r] = quad<T>{};
+            if (r < 2 || k0 + r <= kb) {
+                const unsigned at = __umul24((unsigned)min(k0 + r, kb), (unsigned)N) + (unsigned)cb;
+                vx[r] = *reinterpret_cast<const quad<T>*>(fx + at);
+                vy[r] = *reinterpret_cast<const quad<T>*>(fy + at);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kDirRows; ++r) {
+            if (k0 + r > kb) continue;
+            const T jx = (T)(k0 + r - rv.bxl);
+            const T tx = max(min(rv.xr - jx, (T)1) - max(rv.dx - jx, (T)0), (T)0);
+            T sx_ = (T)0, sy_ = (T)0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                sx_ += tyv[q] * vx[r].v[q];
+                sy_ += tyv[q] * vy[r].v[q];
+            }
+            const size_t row = (size_t)(k0 + r) * N + rv.byl;
+            for (int q = o + 4; q <= rv.ny; ++q) {
+                const T ty = min(rv.yr, (T)(q + 1)) - max(rv.dy, (T)q);
+                if (!(ty > (T)0)) continue;
+                sx_ += ty * fx[row + q];
+                sy_ += ty * fy[row + q];
+            }
+            ax += tx * sx_;
+            ay += tx * sy_;
+        }
+    }
+    const T sc = rv.rat * (T)(g.bsx * g.bsy);
+    return vec2_t<T>{sc * ax, sc * ay};
+}
+
+template <typename T>
+__global__ __launch_bounds__(kDirThreads) void k_gather_cells(
+    const T* __restrict__ px, const T* __restrict__ py, const T* __restrict__ sx,
+    const T* __restrict__ sy, int nc, Grid g, int R, int lgR, const T* __restrict__ fx,
+    const T* __restrict__ fy, T* __restrict__ gx, T* __restrict__ gy)
+{
+    extern __shared__ __align__(16) unsigned char smem[];    // gather_out_lds
+    unsigned* ntall = reinterpret_cast<unsigned*>(smem);
+    unsigned* list = ntall + 1;
+    unsigned* large = list + kDirThreads;
+    double* red = reinterpret_cast<double*>(
+        smem + ((1 + kDirThreads + kDirThreads / 32) * sizeof(unsigned) + 15) / 16 * 16);
+    const int tid = threadIdx.x;
+    if (tid == 0) *ntall = 0u;
+    if (tid < kDirThreads / 32) large[tid] = 0u;
+    __syncthreads();
+    const int i = (int)blockIdx.x * kDirThreads + tid;
+    if (i < nc) {
+        CellSpan c;
+        const bool ok = load_span(px, py, sx, sy, i, g, c);
+        int s0, s1;
+        bool tall = false;
+        if (ok) cell_strips<T>(c, g, R, lgR, s0, s1, tall);
+        tall = tall || (ok && c.byh - c.byl >= kDirCols);
+        if (tall) {
+            list[atomicAdd(ntall, 1u)] = (unsigned)i;
+        } else {
+            const vec2_t<T> v = ok ? cell_force<T>(c, g, fx, fy) : vec2_t<T>{(T)0, (T)0};
+            gx[i] = v.x;
+            gy[i] = v.y;
+        }
+    }
+    __syncthreads();
+    const unsigned n = *ntall;                // uniform across the group
+    if (n == 0u) return;
+    constexpr int kTeams = kDirThreads / kTallTeam;
+    const int team = tid / kTallTeam, lane = tid % kTallTeam;
+    for (unsigned t = team; t < n; t += kTeams)
+        if (!gather_tall_team<T>((int)list[t], lane, px, py, sx, sy, g, fx, fy, gx, gy) &&
+            lane == 0)
+            atomicOr(&large[t >> 5], 1u << (t & 31u));
+    __syncthreads();
+    for (unsigned t = 0; t < n; ++t)          // uniform across the group
+        if ((large[t >> 5] >> (t & 31u)) & 1u)
+            gather_tall<T, kDirThreads>((int)list[t], px, py, sx, sy, g, fx, fy, red, gx, gy);
 }
 
 }  // namespace dpep

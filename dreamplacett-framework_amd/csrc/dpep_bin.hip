@@ -89,8 +89,14 @@ hipError_t launch_bin_gather(const T* px, const T* py, const T* sx,
                              T* gx, T* gy, hipStream_t s, const hipEvent_t* ev)
 {
     if (nc <= 0) return hipSuccess;
-    const size_t lds = gather_lds<T>(b.R, g.N);
     const hipEvent_t* evg1 = ev ? ev + 0 : nullptr;
+    if (gather_direct(g, nc, sizeof(T))) {
+        DPEP_LAUNCH(evg1, (k_gather_cells<T>), (unsigned)((nc + kDirThreads - 1) / kDirThreads),
+                    kDirThreads, (gather_out_lds<kDirThreads, 1>()), s, px, py, sx, sy, nc, g, b.R,
+                    b.lgR, fx, fy, gx, gy);
+        return hipGetLastError();
+    }
+    const size_t lds = gather_lds<T>(b.R, g.N);
     const hipEvent_t* evg2 = ev ? ev + 2 : nullptr;
     if (b.Wgat == b.S)      // one workgroup per strip: item w is mostly strip w
         DPEP_LAUNCH(evg1, (k_gather_bin<T, true>), b.Wgat, kAccThreads, lds, s, g, b, fx, fy);

@@ -319,6 +319,22 @@ inline int run_capacity(long long nc_max)
 // list ~30 per strip; what finds no room goes through the side map.
 constexpr int kTallCap = 512;
 
+// Whether a step gathers each cell's force from the maps themselves
+// (k_gather_cells) instead of per strip (k_gather_bin, k_gather_out).  Step,
+// per strip -> direct, us: float32 512 x 512 78K cells 39.7 -> 38.1, 193K 43.6
+// -> 42.0, 435K 56.7 -> 57.9; 256 x 256 48K 33.2 -> 30.4; 1024 x 1024 (8 MB of
+// fields, twice an XCD's L2) 40K 60.5 -> 56.9, 129K 60.2 -> 59.3 or even,
+// 313K 64.2 -> 67.9; float64 512 x 512 78K 50.1 -> 47.2, 193K 54.9 -> 55.2;
+// 1024 x 1024 40K 73.6 -> 70.0, 129K 75.8 -> 76.7.  So the line lies at a
+// number of cells by the maps' size, half of it where a value is twice as
+// long; larger maps were not measured and keep the strips.
+inline bool gather_direct(const Grid& g, int nc, size_t esz)
+{
+    const size_t mn = (size_t)g.M * g.N;
+    const size_t most = mn <= (1u << 18) ? 768u << 10 : mn <= (1u << 20) ? 384u << 10 : 0;
+    return (size_t)(nc > 0 ? nc : 0) * esz <= most;
+}
+
 struct OnceBlocks {
     int grid;   // blocks (at least one)
     int q;      // cells per block (the last one may hold fewer)

@@ -236,6 +236,7 @@ int run(int M, int N, const Grid& g, int dtype, bool potential, bool gather, int
         (uint4*)sc, n16, M, (T*)(sc + l.twM), (T*)(sc + l.postM), gM, N, (T*)(sc + l.twN),
         (T*)(sc + l.postN), gN);
     NA_TRY(hipGetLastError());
+    if (!gather || gather_direct(g, nc, esz)) b.pos = nullptr;      // G2 alone reads it
     NA_TRY(launch_bin_scatter<T>((const T*)px, (const T*)py, (const T*)sx, (const T*)sy, nc,
                                  g, b, a, d0, (T*)dens, Tt, false, s, nullptr));
     NA_TRY(launch_col_pass<T>(a, Tt, Ux, Uy, s));

@@ -242,7 +242,8 @@ int dpep_get_timings(dpep_ctx* ctx, float* out);
  * launches none and adds 0), [1] strip fill, [2] strip
  * accumulate with the row DCT (and the reduction of split strips),
  * [3] column DCT + inverse, [4] row inverse, [5] gather of the partial
- * forces per strip record, [6] forces in cell order, [7] whole step.
+ * forces per strip record, [6] forces in cell order (where a step of few
+ * cells does both in one kernel, each is half of it), [7] whole step.
  * n = floats in out.  (ABI version 1 had one gather slot at [5] and the
  * step at [6].) */
 int dpep_get_kernel_times(dpep_ctx* ctx, float* out, int n);

@@ -277,6 +277,32 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
                 return hipSuccess;
             });
         }
+        // the direct gather on the same fields (chosen by gather_direct in the
+        // library), against the gather per strip: both sum the same terms,
+        // each within ~20 roundings of it, and a force's terms add up to at
+        // most the cell's area times the largest field value
+        if (nc > 0) {
+            T* dgx = exact<T>(nc);
+            T* dgy = exact<T>(nc);
+            launch((unsigned)((nc + kDirThreads - 1) / kDirThreads), kDirThreads, gather_out_lds<kDirThreads, 1>(), [&] {
+                k_gather_cells<T>(px, py, sx, sy, nc, g, b.R, b.lgR, fx, fy, dgx, dgy);
+            });
+            double mx = 0, my = 0;
+            for (size_t i = 0; i < mn; ++i) {
+                mx = fmax(mx, fabs((double)fx[i]));
+                my = fmax(my, fabs((double)fy[i]));
+            }
+            const double eps = sizeof(T) == 4 ? 0x1p-24 : 0x1p-53;
+            for (int i = 0; i < nc; ++i) {
+                const double area = fmax((double)sx[i] * sy[i], 0.0);
+                if (!(fabs((double)dgx[i] - gx[i]) <= 40 * eps * area * mx) ||
+                    !(fabs((double)dgy[i] - gy[i]) <= 40 * eps * area * my)) {
+                    fprintf(stderr, "direct gather of cell %d: %g %g, per strip %g %g\n", i,
+                            (double)dgx[i], (double)dgy[i], (double)gx[i], (double)gy[i]);
+                    return 4;
+                }
+            }
+        }
         // the older set of counts is zero again for the next step
         const unsigned* older = b.xtot + (size_t)(b.par ^ 1) * nslot;
         for (size_t s2 = 0; s2 < nslot; ++s2)
