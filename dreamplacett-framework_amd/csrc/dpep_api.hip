@@ -94,6 +94,7 @@ struct dpep_ctx {
     void* d_raw = nullptr;       // scatter density without D0 (DPEP_FLAG_SCATTER_DENSITY)
     BinPlan plan{};
     BinArgs bins{};
+    void* d_strips = nullptr;    // the per-strip state of bins, one allocation
     void *d_twM = nullptr, *d_postM = nullptr, *d_twN = nullptr,
          *d_postN = nullptr;
     hipStream_t stream = nullptr;
@@ -164,10 +165,8 @@ static void release(dpep_ctx* c)
     void* bufs[] = {c->d_px, c->d_py, c->d_sx, c->d_sy, c->d_d0n,
                     c->d_density, c->d_potential, c->d_fx, c->d_fy, c->d_gx,
                     c->d_gy, c->d_T, c->d_Ux, c->d_Uy, c->d_twM,
-                    c->d_postM, c->d_twN, c->d_postN, b.cnt, b.xtot, b.pbase,
-                    b.pcap, b.pool_n, b.ovst, b.oruns, b.items, b.nitems, b.done, b.recg,
-                    b.recm, b.pos, b.gtmp,
-                    b.bigflag, b.B, b.chunk, b.items_g, b.tall_n, b.tall_cell, c->d_raw};
+                    c->d_postM, c->d_twN, c->d_postN, c->d_strips, b.recg, b.recm, b.pos,
+                    b.gtmp, b.B, c->d_raw};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     for (auto& e : c->ev)
@@ -395,44 +394,52 @@ int dpep_create(int M, int N, int nc_max, double xl, double yl, double xh,
                                           c->device));
             set_item_grids(b, acc, gat, cus);
         }
-        HIP_TRY(hipMalloc((void**)&b.cnt, (size_t)p.G1max * p.S * sizeof(unsigned)));
-        // two sets of (slot, strip) counts: this step's and the last one's
-        HIP_TRY(hipMalloc((void**)&b.xtot, 2 * (size_t)kCountSlots * p.S * sizeof(unsigned)));
-        HIP_TRY(hipMemset(b.xtot, 0, 2 * (size_t)kCountSlots * p.S * sizeof(unsigned)));
-        HIP_TRY(hipMalloc((void**)&b.pbase, (size_t)kCountSlots * p.S * sizeof(unsigned)));
-        HIP_TRY(hipMalloc((void**)&b.pcap, (size_t)kCountSlots * p.S * sizeof(unsigned)));
-        HIP_TRY(hipMalloc((void**)&b.pool_n, 2 * sizeof(unsigned)));
-        HIP_TRY(hipMemset(b.pool_n, 0, 2 * sizeof(unsigned)));
         // records: the plan's regions, then an overflow pool of one slot per
         // possible record
         b.reg_cap = (unsigned)p.reg_cap;
         b.pool0 = (unsigned)p.reg_cap;
         b.pool_cap = (unsigned)p.cap;
         const size_t nrec = p.reg_cap + p.cap;
-        HIP_TRY(hipMalloc((void**)&b.ovst, 2 * (size_t)p.S * sizeof(unsigned long long)));
-        HIP_TRY(hipMemset(b.ovst, 0, 2 * (size_t)p.S * sizeof(unsigned long long)));
         b.rmax = run_capacity(nc_max);
-        HIP_TRY(hipMalloc((void**)&b.oruns, (size_t)p.S * b.rmax * sizeof(uint2)));
-        HIP_TRY(hipMalloc((void**)&b.items, (size_t)b.Wacc * sizeof(uint4)));
-        HIP_TRY(hipMalloc((void**)&b.items_g, (size_t)b.Wgat * sizeof(uint4)));
-        HIP_TRY(hipMalloc((void**)&b.nitems, 2 * sizeof(unsigned)));
-        HIP_TRY(hipMalloc((void**)&b.chunk, 2 * sizeof(unsigned)));
-        HIP_TRY(hipMalloc((void**)&b.done, (size_t)p.S * sizeof(unsigned)));
-        HIP_TRY(hipMemset(b.done, 0, (size_t)p.S * sizeof(unsigned)));
+        b.tall_cap = kTallCap;
+        // the per-strip state in one allocation (each costs ~0.1 ms or more),
+        // what must start at zero first: two sets of (slot, strip) counts (this
+        // step's and the last one's), of overflow and of tall-list state, the
+        // strip flags and chunk counters, which each step leaves at zero
+        const size_t S = (size_t)p.S, u = sizeof(unsigned);
+        struct { void** at; size_t bytes; } parts[] = {
+            {(void**)&b.xtot, 2 * kCountSlots * S * u}, {(void**)&b.pool_n, 2 * u},
+            {(void**)&b.ovst, 2 * S * sizeof(unsigned long long)},
+            {(void**)&b.tall_n, 2 * S * u}, {(void**)&b.done, S * u},
+            {(void**)&b.bigflag, kSideWords * S * u},
+            {(void**)&b.cnt, (size_t)p.G1max * S * u}, {(void**)&b.pbase, kCountSlots * S * u},
+            {(void**)&b.pcap, kCountSlots * S * u},
+            {(void**)&b.oruns, S * (size_t)b.rmax * sizeof(uint2)},
+            {(void**)&b.items, (size_t)b.Wacc * sizeof(uint4)},
+            {(void**)&b.items_g, (size_t)b.Wgat * sizeof(uint4)},
+            {(void**)&b.nitems, 2 * u}, {(void**)&b.chunk, 2 * u},
+            {(void**)&b.tall_cell, S * kTallCap * 4 * c->esz}};
+        constexpr int kZeroParts = 6;
+        size_t bytes = 0, zero = 0;
+        int k = 0;
+        for (auto& q : parts) {
+            bytes += (q.bytes + 255) / 256 * 256;
+            if (++k == kZeroParts) zero = bytes;
+        }
+        HIP_TRY(hipMalloc(&c->d_strips, bytes));
+        HIP_TRY(hipMemset(c->d_strips, 0, zero));
+        char* at = (char*)c->d_strips;
+        for (auto& q : parts) {
+            *q.at = at;
+            at += (q.bytes + 255) / 256 * 256;
+        }
         HIP_TRY(hipMalloc(&b.recg, nrec * p.geo_bytes));
         HIP_TRY(hipMalloc((void**)&b.recm, (p.span_bytes ? nrec : 1) * sizeof(unsigned)));
         HIP_TRY(hipMalloc((void**)&b.pos, (size_t)(nc_max > 0 ? nc_max : 1) * sizeof(unsigned long long)));
         HIP_TRY(hipMalloc(&b.gtmp, nrec * 2 * c->esz));
-        HIP_TRY(hipMalloc((void**)&b.bigflag, (size_t)kSideWords * p.S * sizeof(unsigned)));
+        // B must start at zero; each step leaves it so
         HIP_TRY(hipMalloc(&b.B, (size_t)M * N * accb));
-        // per-strip lists of tall cells
-        b.tall_cap = kTallCap;
-        HIP_TRY(hipMalloc((void**)&b.tall_n, 2 * (size_t)p.S * sizeof(unsigned)));
-        HIP_TRY(hipMemset(b.tall_n, 0, 2 * (size_t)p.S * sizeof(unsigned)));
-        HIP_TRY(hipMalloc(&b.tall_cell, (size_t)p.S * kTallCap * 4 * c->esz));
-        // B and the strip flags must start at zero; each step leaves them so.
         HIP_TRY(hipMemset(b.B, 0, (size_t)M * N * accb));
-        HIP_TRY(hipMemset(b.bigflag, 0, (size_t)kSideWords * p.S * sizeof(unsigned)));
         HIP_TRY(hipDeviceSynchronize());
         return dtype == DPEP_DTYPE_F32 ? make_tables<float>(c) : make_tables<double>(c);
     };
