@@ -12,7 +12,7 @@
 //   k_bin_fill    each workgroup scans the strip totals for its own   K3
 //                 offsets (a workgroup of its own publishes the strip
 //                 table, the chunk sizes and the K4 / G1 item lists);
-//                 cells -> strip-sorted records; tall cells -> B
+//                 cells -> strip-sorted records; tall cells -> lists
 //                 (K1 and this form: the first step, or every step
 //                 with DPEP_FLAG_TWO_PASS; each one-pass block split
 //                 into counting parts of at most 1024 cells)
@@ -53,9 +53,9 @@
 // forces in cell order instead of G1 scattering them.
 //
 // A cell whose span covers more than R rows or more than kMaxSpanY + 1
-// columns ("tall") skips the sort.  The one-pass K3 enters it in the list of
-// every strip it touches and K4 adds its bins in the strip's LDS tile
-// (list_tall_team); a counted K3, and a list that is full, adds it with global
+// columns ("tall") skips the sort.  K3 enters it in the list of every strip
+// it touches and K4 adds its bins in the strip's LDS tile (list_tall); where
+// a list is full, or there are none (the no-alloc step), K3 adds it with global
 // atomics into the side map B (zero between steps) and marks the column blocks
 // it touches in each of its strips, and K4 folds and re-zeroes those blocks
 // of B.  G2 gathers the cell with a team of threads.  Every other cell touches at most
@@ -340,17 +340,22 @@ __device__ __forceinline__ void load_cells(const T* __restrict__ px, const T* __
     }
 }
 
-// The cells [c0, cend) of counting workgroup blockIdx.x (K1, the fresh K3:
-// part blockIdx.x % b.sub of one-pass block blockIdx.x / b.sub, see
-// set_count_blocks) and its count slot, the one-pass block's.
-__device__ __forceinline__ int count_cells(const BinArgs& b, int nc, int& c0, int& cend)
+// The cells [c0, cend) of counting workgroup w (K1, the fresh K3: part
+// w % b.sub of one-pass block w / b.sub, see set_count_blocks) and its count
+// slot, the one-pass block's.
+__device__ __forceinline__ int group_cells(const BinArgs& b, int w, int nc, int& c0, int& cend)
 {
-    const int ob = (int)blockIdx.x / b.sub, part = (int)blockIdx.x - ob * b.sub;
+    const int ob = w / b.sub, part = w - ob * b.sub;
     const int base = ob * b.qcells;
     c0 = base + part * b.qsub;
     cend = min(min(c0 + b.qsub, base + b.qcells), nc);
     if (cend < c0) cend = c0;
     return ob & (kCountSlots - 1);
+}
+
+__device__ __forceinline__ int count_cells(const BinArgs& b, int nc, int& c0, int& cend)
+{
+    return group_cells(b, (int)blockIdx.x, nc, c0, cend);       // K1
 }
 
 // The CPT cells of thread tid in the one-pass block [c0, cend) (slots past
@@ -549,19 +554,28 @@ __device__ __forceinline__ void publish_items(const BinArgs& b, const unsigned* 
 // a few microseconds of L2 reads spread over the grid) instead of one
 // workgroup building a table behind all of K1.  The regions of a strip are
 // its slots' totals back to back, exactly: cur[s] = strip offset + totals
-// of the slots before g's + g's base within its slot.  The last workgroup,
-// one past those that hold cells, also publishes the plan for K4 / G1 (the
-// no-alloc step at 150K cells on 512 x 512: 48.4 -> 46.8 us against the
-// first workgroup doing it before its cells).  LDS: cur[S] | tot[S] | tmp[kBinThreads]
+// of the slots before g's + g's base within its slot.  The grid begins with
+// kPlanGroups workgroups that hold no cells: the first publishes the plan for
+// K4 / G1, the others return, so the workgroups of cells keep K1's XCDs (the
+// no-alloc step at 150K cells on 512 x 512: 48.4 -> 46.8 us against the first
+// workgroup of cells doing it before its cells; by one past the last, which
+// starts after a full round of others, 1.1M cells counted on 2048 x 2048 took
+// 114.4 -> 116.1, at the front no longer than before).  LDS: cur[S] | tot[S] | tmp[kBinThreads]
 // | cand[kChunkCands].
+__device__ __forceinline__ int fill_group()    // the planning one: past all cells
+{
+    return (int)(blockIdx.x == 0u ? gridDim.x : blockIdx.x) - kPlanGroups;
+}
+
 __device__ __forceinline__ void fresh_offsets(const BinArgs& b, unsigned* cur,
                                               unsigned* tot, unsigned* tmp)
 {
     const int tid = threadIdx.x;
     const int S = b.S;
     int c0, cend;
-    const int x = count_cells(b, 0, c0, cend);
-    const unsigned* row = b.cnt + (size_t)blockIdx.x * S;
+    const int w = fill_group();
+    const int x = group_cells(b, w, 0, c0, cend);
+    const unsigned* row = b.cnt + (size_t)w * S;
     const unsigned* xt = counts_of(b, b.par);
     for (int s = tid; s < S; s += kBinThreads) {
         unsigned t = 0u, pre = 0u;
@@ -582,7 +596,7 @@ __device__ __forceinline__ void fresh_offsets(const BinArgs& b, unsigned* cur,
     for (int s = r0; s < r1; ++s) run += tot[s];
     unsigned total;
     unsigned base = block_exclusive_scan(run, tmp, total);
-    const bool pub = blockIdx.x == gridDim.x - 1u;   // uniform across the group
+    const bool pub = blockIdx.x == 0u;        // uniform across the group
     for (int s = r0; s < r1; ++s) {
         cur[s] += base;
         if (pub) {
@@ -598,6 +612,93 @@ __device__ __forceinline__ void fresh_offsets(const BinArgs& b, unsigned* cur,
         base += tot[s];
     }
     if (pub) publish_items(b, tot, tmp, r0, r1);
+}
+
+// Threads per team that handles one tall cell (K3's side-map adds, G2's
+// gather).
+constexpr int kTallTeam = 16;
+
+// A tall cell's density over rows [ka, kb], one value per bin, by a team of W
+// threads (lane: index in the team; every lane calls it for the same
+// cell): add(row, column, fixed-point value) for the bins strided over the
+// team.  Each is the value a single thread's row-by-row loop adds, (ratio /
+// bin area * tx) * ty in fixed point, so the sums are bitwise the same in any
+// order and whether B or a strip's LDS tile receives them.  One thread per
+// tall cell held its workgroup ~10 us for a cell of ~50 bins (float64).
+template <int W = kTallTeam, typename Fn>
+__device__ __forceinline__ void tall_density(const CellSpan& c, int ka, int kb, int lane,
+                                             const Grid& g, Fn&& add)
+{
+    const double sc = c.ratio() * g.inv_ba;
+    const int ny1 = c.byh - c.byl + 1;
+    const int nb = (kb - ka + 1) * ny1;
+    for (int e = lane; e < nb; e += W) {
+        const int k = ka + e / ny1, q = c.byl + e % ny1;
+        const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
+        const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
+        if (tx <= 0.0 || ty <= 0.0) continue;
+        const double stx = sc * tx;
+        add(k, q, to_fixed(stx * ty, g.fix_scale));
+    }
+}
+
+// One tall cell, by a team of W threads (in a counted K3 its own thread): an entry
+// in the list of every strip it touches, from which K4 adds its bins in the
+// strip's LDS tile.  A strip whose list is full takes the cell's bins in its
+// rows through the side map B instead (marked for K4's fold), and so do all
+// strips of a cell of more than kTallStrips strips or kTallBins bins in a
+// strip (a team would walk it for long).  The sums are bitwise the same.
+// Through B, a strip with any tall cell pays a dependent round of loads in K4
+// and a read and a rewrite of the marked blocks of 64-bit words: 12 K tall
+// cells of 2.0 M on 4096 x 4096 (a quarter of B marked) K4 104.7 -> 82.0 us and
+// K3 54.8 -> 52.7, ~300 of 210 K on 2048 x 2048 step 99.2 -> 95.  On a counted
+// step, whose K3 added a tall cell's ~50 bins by its one thread: step on 4096 x
+// 4096 447 -> 396, 600 K on 2048 x 2048 102.7 -> 97.6.  (Gathering
+// them in G1 the same way, partials per strip summed by G2, made G1 11 us
+// slower at 4096 x 4096 against 2 us won in G2.)
+constexpr int kTallStrips = 32;
+constexpr int kTallBins = 512;
+
+template <typename T, int W>
+__device__ __forceinline__ void list_tall(const vec4_t<T>& cell, const CellSpan& c, int s0, int s1,
+                                          int lane, const Grid& g, const BinArgs& b,
+                                          unsigned long long* __restrict__ Bm)
+{
+    unsigned refused = ~0u;                     // bit j: strip s0 + j
+    if (b.tall_n && s1 - s0 < kTallStrips && b.R * (c.byh - c.byl + 1) <= kTallBins) {
+        refused = 0u;
+        for (int s = s0 + lane; s <= s1; s += W) {
+            const unsigned e = atomicAdd(&b.tall_n[(size_t)(b.par & 1) * b.S + s], 1u);
+            if (e < b.tall_cap)
+                reinterpret_cast<vec4_t<T>*>(b.tall_cell)[(size_t)s * b.tall_cap + e] = cell;
+            else
+                refused |= 1u << (s - s0);
+        }
+#pragma unroll
+        for (int m = W / 2; m > 0; m >>= 1) refused |= __shfl_xor(refused, m, W);
+        if (refused == 0u) return;              // uniform across the team
+    }
+    auto through_b = [&](int s) { return s - s0 >= kTallStrips || ((refused >> (s - s0)) & 1u); };
+    tall_density<W>(c, c.bxl, c.bxh, lane, g, [&](int k, int q, unsigned long long v) {
+        if (through_b(k >> b.lgR)) atomicAdd(&Bm[(size_t)k * g.N + q], v);
+    });
+    const int CB = side_block(g.N);
+    for (int s = s0 + lane; s <= s1; s += W)
+        if (through_b(s)) side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
+}
+
+template <typename T>
+__device__ __forceinline__ void list_tall_team(const vec4_t<T>& cell, int lane,
+                                               const Grid& g, const BinArgs& b,
+                                               unsigned long long* __restrict__ Bm)
+{
+    CellSpan c;
+    if (!cell_span((double)cell.x, (double)cell.y, (double)cell.z, (double)cell.w, g, c))
+        return;
+    int s0, s1;
+    bool tall;
+    cell_strips<T>(c, g, b.R, b.lgR, s0, s1, tall);
+    list_tall<T, kTallTeam>(cell, c, s0, s1, lane, g, b, Bm);
 }
 
 // Capacity a one-pass step gives a region that counted d records in the
@@ -842,11 +943,12 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_fill_direct(
     BinArgs b)
 {
     extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x > 0u && blockIdx.x < (unsigned)kPlanGroups) return;
     unsigned* cur = reinterpret_cast<unsigned*>(smem);
     const int tid = threadIdx.x;
     // the cells' loads are issued first: their latency overlaps the offsets
     int c0, cend;
-    count_cells(b, nc, c0, cend);
+    group_cells(b, fill_group(), nc, c0, cend);
     T cx[kCellsPerThread], cy[kCellsPerThread], cw[kCellsPerThread], chh[kCellsPerThread];
     load_cells(px, py, sx, sy, cend, c0, tid, cx, cy, cw, chh);
     fresh_offsets(b, cur, cur + b.S, cur + 2 * b.S);
@@ -865,22 +967,7 @@ __global__ __launch_bounds__(kBinThreads) void k_bin_fill_direct(
         bool tall;
         cell_strips<T>(c, g, b.R, b.lgR, s0, s1, tall);
         if (tall) {
-            const double sc = c.ratio() * g.inv_ba;
-            for (int k = c.bxl; k <= c.bxh; ++k) {
-                const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
-                if (tx <= 0.0) continue;
-                const double stx = sc * tx;
-                const size_t rowi = (size_t)k * g.N;
-                for (int q = c.byl; q <= c.byh; ++q) {
-                    const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
-                    if (ty <= 0.0) continue;
-                    atomicAdd(&Bm[rowi + q], to_fixed(stx * ty, g.fix_scale));
-                }
-            }
-            // the column blocks of B this cell touches, in each of its strips
-            const int CB = side_block(g.N);
-            for (int s = s0; s <= s1; ++s)
-                side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
+            list_tall<T, 1>(vec4_t<T>{cx[j], cy[j], cw[j], chh[j]}, c, s0, s1, 0, g, b, Bm);
             put_pos(b, i, pos_pair(kPosTall, kPosNone));
             continue;
         }
@@ -942,6 +1029,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
     BinArgs b)
 {
     extern __shared__ __align__(16) unsigned char smem[];
+    if (blockIdx.x > 0u && blockIdx.x < (unsigned)kPlanGroups) return;
     const int S = b.S;
     unsigned* cur = reinterpret_cast<unsigned*>(smem);
     unsigned* cnt = cur + S;              // strip totals, then this block's counts
@@ -954,7 +1042,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
     const int tid = threadIdx.x;
     // the cells' loads are issued first: their latency overlaps the offsets
     int c0, cend;
-    count_cells(b, nc, c0, cend);
+    group_cells(b, fill_group(), nc, c0, cend);
     T cx[kCellsPerThread], cy[kCellsPerThread], cw[kCellsPerThread], chh[kCellsPerThread];
     load_cells(px, py, sx, sy, cend, c0, tid, cx, cy, cw, chh);
     fresh_offsets(b, cur, cnt, tmp);
@@ -983,22 +1071,7 @@ __global__ __launch_bounds__(kBinThreads, 5) void k_bin_fill_staged(
         bool tall;
         cell_strips<T>(c, g, b.R, b.lgR, s0, s1, tall);
         if (tall) {
-            const double sc = c.ratio() * g.inv_ba;
-            for (int k = c.bxl; k <= c.bxh; ++k) {
-                const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
-                if (tx <= 0.0) continue;
-                const double stx = sc * tx;
-                const size_t rowi = (size_t)k * g.N;
-                for (int q = c.byl; q <= c.byh; ++q) {
-                    const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
-                    if (ty <= 0.0) continue;
-                    atomicAdd(&Bm[rowi + q], to_fixed(stx * ty, g.fix_scale));
-                }
-            }
-            // the column blocks of B this cell touches, in each of its strips
-            const int CB = side_block(g.N);
-            for (int s = s0; s <= s1; ++s)
-                side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
+            list_tall<T, 1>(vec4_t<T>{cx[j], cy[j], cw[j], chh[j]}, c, s0, s1, 0, g, b, Bm);
             put_pos(b, i, pos_pair(kPosTall, kPosNone));
             continue;
         }
@@ -1126,83 +1199,6 @@ __device__ __forceinline__ void record_density(const vec4_t<T>& rg, unsigned rm,
         density_rows<T, 4>(rv, tyv, ka, kb, k0, N, fs, tile);
     else
         density_rows<T, 3>(rv, tyv, ka, kb, k0, N, fs, tile);
-}
-
-// Threads per team that handles one tall cell (K3's side-map adds, G2's
-// gather).
-constexpr int kTallTeam = 16;
-
-// A tall cell's density over rows [ka, kb], one value per bin, by a team of
-// kTallTeam threads (lane: index in the team; every lane calls it for the same
-// cell): add(row, column, fixed-point value) for the bins strided over the
-// team.  Each is the value a single thread's row-by-row loop adds, (ratio /
-// bin area * tx) * ty in fixed point, so the sums are bitwise the same in any
-// order and whether B or a strip's LDS tile receives them.  One thread per
-// tall cell held its workgroup ~10 us for a cell of ~50 bins (float64).
-template <typename Fn>
-__device__ __forceinline__ void tall_density(const CellSpan& c, int ka, int kb, int lane,
-                                             const Grid& g, Fn&& add)
-{
-    const double sc = c.ratio() * g.inv_ba;
-    const int ny1 = c.byh - c.byl + 1;
-    const int nb = (kb - ka + 1) * ny1;
-    for (int e = lane; e < nb; e += kTallTeam) {
-        const int k = ka + e / ny1, q = c.byl + e % ny1;
-        const double tx = overlap_1d(c.x, c.w, g.xl, g.bsx, k);
-        const double ty = overlap_1d(c.y, c.h, g.yl, g.bsy, q);
-        if (tx <= 0.0 || ty <= 0.0) continue;
-        const double stx = sc * tx;
-        add(k, q, to_fixed(stx * ty, g.fix_scale));
-    }
-}
-
-// One tall cell of a one-pass step, by a team of kTallTeam threads: an entry
-// in the list of every strip it touches, from which K4 adds its bins in the
-// strip's LDS tile.  A strip whose list is full takes the cell's bins in its
-// rows through the side map B instead (marked for K4's fold), and so do all
-// strips of a cell of more than kTallStrips strips or kTallBins bins in a
-// strip (a team would walk it for long).  The sums are bitwise the same.
-// Through B, a strip with any tall cell pays a dependent round of loads in K4
-// and a read and a rewrite of the marked blocks of 64-bit words: 12 K tall
-// cells of 2.0 M on 4096 x 4096 (a quarter of B marked) K4 104.7 -> 82.0 us and
-// K3 54.8 -> 52.7, ~300 of 210 K on 2048 x 2048 step 99.2 -> 95.  (Gathering
-// them in G1 the same way, partials per strip summed by G2, made G1 11 us
-// slower at 4096 x 4096 against 2 us won in G2.)
-constexpr int kTallStrips = 32;
-constexpr int kTallBins = 512;
-
-template <typename T>
-__device__ __forceinline__ void list_tall_team(const vec4_t<T>& cell, int lane,
-                                               const Grid& g, const BinArgs& b,
-                                               unsigned long long* __restrict__ Bm)
-{
-    CellSpan c;
-    if (!cell_span((double)cell.x, (double)cell.y, (double)cell.z, (double)cell.w, g, c))
-        return;
-    int s0, s1;
-    bool tall;
-    cell_strips<T>(c, g, b.R, b.lgR, s0, s1, tall);
-    unsigned refused = ~0u;                     // bit j: strip s0 + j
-    if (b.tall_n && s1 - s0 < kTallStrips && b.R * (c.byh - c.byl + 1) <= kTallBins) {
-        refused = 0u;
-        for (int s = s0 + lane; s <= s1; s += kTallTeam) {
-            const unsigned e = atomicAdd(&b.tall_n[(size_t)(b.par & 1) * b.S + s], 1u);
-            if (e < b.tall_cap)
-                reinterpret_cast<vec4_t<T>*>(b.tall_cell)[(size_t)s * b.tall_cap + e] = cell;
-            else
-                refused |= 1u << (s - s0);
-        }
-#pragma unroll
-        for (int m = kTallTeam / 2; m > 0; m >>= 1) refused |= __shfl_xor(refused, m, kTallTeam);
-        if (refused == 0u) return;              // uniform across the team
-    }
-    auto through_b = [&](int s) { return s - s0 >= kTallStrips || ((refused >> (s - s0)) & 1u); };
-    tall_density(c, c.bxl, c.bxh, lane, g, [&](int k, int q, unsigned long long v) {
-        if (through_b(k >> b.lgR)) atomicAdd(&Bm[(size_t)k * g.N + q], v);
-    });
-    const int CB = side_block(g.N);
-    for (int s = s0 + lane; s <= s1; s += kTallTeam)
-        if (through_b(s)) side_mark(b.bigflag + (size_t)s * kSideWords, c.byl, c.byh, CB);
 }
 
 // ---------------------------------------------------------------------------

@@ -65,12 +65,12 @@ hipError_t launch_bin_scatter(const T* px, const T* py, const T* sx,
         DPEP_LAUNCH(ev1, (k_bin_count<T>), b.G1, kBinThreads, count_lds, s, px, py, sx, sy,
                     nc, g, b);
         if ((e = hipGetLastError())) return e;
-        // one workgroup past the cells' publishes the plan
+        // the first workgroup publishes the plan
         if (staged)
-            DPEP_LAUNCH(ev3, (k_bin_fill_staged<T>), b.G1 + 1, kBinThreads, fill_lds, s, px, py, sx,
+            DPEP_LAUNCH(ev3, (k_bin_fill_staged<T>), b.G1 + kPlanGroups, kBinThreads, fill_lds, s, px, py, sx,
                         sy, nc, g, b);
         else
-            DPEP_LAUNCH(ev3, (k_bin_fill_direct<T>), b.G1 + 1, kBinThreads, fill_lds, s, px, py, sx,
+            DPEP_LAUNCH(ev3, (k_bin_fill_direct<T>), b.G1 + kPlanGroups, kBinThreads, fill_lds, s, px, py, sx,
                         sy, nc, g, b);
     }
     if ((e = hipGetLastError())) return e;

@@ -114,8 +114,8 @@ constexpr unsigned kRegionSlack = 16;
 // Records live in kCountSlots regions per strip (workgroup g reserves its
 // runs in region g % kCountSlots of each strip: the reservation atomics are
 // spread over kCountSlots counters per strip).  K3's last workgroup, which
-// holds no cells, publishes the step's plan: where the regions are (pbase, pcap) and the K4 / G1 work
-// items.  Within a strip the records are numbered region after region,
+// holds no cells (a counted K3's first), publishes the step's plan: where the
+// regions are (pbase, pcap) and the K4 / G1 work items.  Within a strip the records are numbered region after region,
 // without the unfilled tail of each region ("strip-relative" numbers).  Two
 // ways to fill:
 //   fresh  K1 counts every (slot, strip) first; K3 places the regions
@@ -178,8 +178,8 @@ struct BinArgs {
                             // (zero between steps)
     void* B;                // [M*N] uint64, zero between steps: tall cells and
                             // the chunks of split strips add into it
-    // tall cells of a one-pass step, per strip they touch (null: none, every
-    // tall cell through B, as on a counted step)
+    // tall cells, per strip they touch (null: no lists, every tall cell
+    // through B)
     unsigned* tall_n;       // [2][S] entries of the strip, the step of each parity
                             // (counts the refused ones too; the older set zero
                             // again after K4)
@@ -235,6 +235,10 @@ inline size_t region_capacity(size_t cap, int S)
 {
     return cap + cap / 8 + (size_t)kRegionSlack * kCountSlots * (size_t)S;
 }
+
+// Workgroups of a counted K3 before those that hold cells: the planning one,
+// and idle ones so that the others keep their XCDs (workgroup number % 8).
+constexpr int kPlanGroups = 8;
 
 // Rows of BinArgs::cnt: an upper bound of the counting workgroups
 // (set_count_blocks) of any step of at most nc cells, and one more (K3's

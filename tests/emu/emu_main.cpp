@@ -238,10 +238,10 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
         } else {
             launch(b.G1, kBinThreads, hist, [&] { k_bin_count<T>(px, py, sx, sy, nc, g, b); });
             if (stage)
-                launch(b.G1 + 1, kBinThreads, fill_lds_staged<T>(p.S),
+                launch(b.G1 + kPlanGroups, kBinThreads, fill_lds_staged<T>(p.S),
                        [&] { k_bin_fill_staged<T>(px, py, sx, sy, nc, g, b); });
             else
-                launch(b.G1 + 1, kBinThreads,
+                launch(b.G1 + kPlanGroups, kBinThreads,
                        (size_t)(2 * p.S + kBinThreads + kChunkCands) * sizeof(unsigned),
                        [&] { k_bin_fill_direct<T>(px, py, sx, sy, nc, g, b); });
         }
@@ -322,16 +322,26 @@ static int run(int nc, bool det, bool pot, int ch, bool tall, bool force_stage, 
     // from step 1's counts (no overflow: same cells); step 3 sizes them at
     // half of step 2's counts, so it overflows about half its records --
     // and must give bitwise step 2's results
+    // (a counted step without tall lists first: every tall cell through B)
+    unsigned* const lists = b.tall_n;
+    b.tall_n = nullptr;
     int rc = step(false);
+    b.tall_n = lists;
     if (rc) return rc;
     const std::vector<T> frho(dens, dens + mn), fgx(gx, gx + nc), fgy(gy, gy + nc);
     if (pool_seen) { fprintf(stderr, "fresh step used the pool\n"); return 4; }
+    auto same = [&] {
+        return !memcmp(frho.data(), dens, mn * sizeof(T)) &&
+               !memcmp(fgx.data(), gx, nc * sizeof(T)) && !memcmp(fgy.data(), gy, nc * sizeof(T));
+    };
+    rc = step(false);
+    if (rc) return rc;
+    if (!same()) { fprintf(stderr, "counted step with tall lists differs\n"); return 4; }
     rc = step(true);
     if (rc) return rc;
     if (pool_seen) { fprintf(stderr, "one-pass step on the same cells overflowed (%u)\n", pool_seen); return 4; }
-    // the counted step's tall cells all went through B
-    if (memcmp(frho.data(), dens, mn * sizeof(T)) || memcmp(fgx.data(), gx, nc * sizeof(T)) ||
-        memcmp(fgy.data(), gy, nc * sizeof(T))) {
+    // the first step's tall cells all went through B
+    if (!same()) {
         fprintf(stderr, "one-pass step differs from the counted one\n");
         return 4;
     }
