@@ -325,17 +325,18 @@ constexpr int kTallCap = 512;
 
 // Whether a step gathers each cell's force from the maps themselves
 // (k_gather_cells) instead of per strip (k_gather_bin, k_gather_out).  Step,
-// per strip -> direct, us: float32 512 x 512 78K cells 39.7 -> 38.1, 193K 43.6
-// -> 42.0, 435K 56.7 -> 57.9; 256 x 256 48K 33.2 -> 30.4; 1024 x 1024 (8 MB of
-// fields, twice an XCD's L2) 40K 60.5 -> 56.9, 129K 60.2 -> 59.3 or even,
-// 313K 64.2 -> 67.9; float64 512 x 512 78K 50.1 -> 47.2, 193K 54.9 -> 55.2;
-// 1024 x 1024 40K 73.6 -> 70.0, 129K 75.8 -> 76.7.  So the line lies at a
-// number of cells by the maps' size, half of it where a value is twice as
-// long; larger maps were not measured and keep the strips.
+// per strip -> direct, us, clustered cells: float32 512 x 512 98K cells 38.6 ->
+// 37.4, 262K 47.4 -> 45.7, 350K 53.4 -> 52.2, 435K 56.7 -> 57.9; 256 x 256 260K
+// 45.4 -> 43.3; 1024 x 1024 (8 MB of fields, twice an XCD's L2) 60K 60.3 -> 56.6,
+// 98K 60.0 -> 58.5, 130K 59.1 -> 58.7 (uniform 59.2 -> 59.4), 313K 64.2 -> 67.9;
+// float64 512 x 512 131K 50.8 -> 49.1, 150K even, 193K 54.9 -> 55.2; 1024 x 1024
+// 49K 74.0 -> 70.7, 90K even.  So the line lies at the bytes of one coordinate
+// of the cells, by the maps' size; larger maps were not measured and keep the
+// strips.
 inline bool gather_direct(const Grid& g, int nc, size_t esz)
 {
     const size_t mn = (size_t)g.M * g.N;
-    const size_t most = mn <= (1u << 18) ? 768u << 10 : mn <= (1u << 20) ? 384u << 10 : 0;
+    const size_t most = mn <= (1u << 18) ? 1024u << 10 : mn <= (1u << 20) ? 448u << 10 : 0;
     return (size_t)(nc > 0 ? nc : 0) * esz <= most;
 }
 

@@ -1,6 +1,6 @@
 """GPU: the direct gather (few cells on small maps: one thread per cell reads
 the field bins) and the gather per strip, on either side of the line between
-them (cells times bytes per value: 768 KiB up to 2^18 bins, 384 KiB up to 2^20,
+them (cells times bytes per value: 1 MiB up to 2^18 bins, 448 KiB up to 2^20,
 none beyond), with cells of one to 40 columns and tall ones, on a moving
 placement, against the float64 oracle (the relative error of a field is ~4e-7
 at float32 and ~6e-14 at float64, and a force sums ~10 of its values)."""
@@ -11,9 +11,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("cells,M,N,dtype", [
-    (196608, 512, 512, np.float32), (196609, 512, 512, np.float32),
-    (98304, 256, 1024, np.float64), (98305, 256, 1024, np.float64),
-    (98304, 1024, 1024, np.float32), (98305, 1024, 1024, np.float32),
+    (262144, 512, 512, np.float32), (262145, 512, 512, np.float32),
+    (131072, 256, 1024, np.float64), (131073, 256, 1024, np.float64),
+    (114688, 1024, 1024, np.float32), (114689, 1024, 1024, np.float32),
     (255, 8, 8, np.float32), (257, 8, 32, np.float64), (3000, 4096, 64, np.float32)])
 def test_gather_paths_at_their_line(oracle, cells, M, N, dtype):
     import dpep
