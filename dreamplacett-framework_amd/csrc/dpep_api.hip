@@ -8,7 +8,8 @@
 //                                         and P1 (row DCT) of each strip
 //   k_col_pass  P2
 //   k_row_inv   P3  -> field_x, field_y, potential
-//   k_gather_bin, k_gather_out   per-cell forces <- fields
+//   k_gather_bin, k_gather_out   per-cell forces <- fields (few cells on
+//   or k_gather_cells            small maps: one kernel)
 #include <math.h>
 #include <signal.h>
 #include <stdarg.h>
@@ -788,7 +789,7 @@ int dpep_step_staged(dpep_ctx* c, const void* const cells[4], void* const cell_s
     if (!cells || !cell_stage || !outputs || !output_stage)
         return fail(DPEP_ERR_ARG, "an array of pointers is NULL");
     if (int rc = check_cells(c, cells[0], cells[1], cells[2], cells[3], nc)) return rc;
-    const bool keep_sizes = !cells[2];
+    const bool keep_sizes = !cells[2] && !cells[3];
     const int nin = nc == 0 ? 0 : keep_sizes ? 2 : 4;
     for (int i = 0; i < nin; ++i)
         if (!cell_stage[i]) return fail(DPEP_ERR_ARG, "cell staging buffer is NULL");

@@ -33,6 +33,8 @@
 //                 partials, on the one-pass blocks; tall cells
 //                 gathered by 16-thread teams (larger ones by the
 //                 whole workgroup)
+//   k_gather_cells  few cells on small maps: both of these at once,  G
+//                 a thread per cell reading the maps (gather_direct)
 //
 // Accumulation is fixed point everywhere: round(v * 2^f) added as uint64
 // (LDS, the side map B), with f = fix_exponent_of(nc_max, dtype) so a bin's
@@ -642,8 +644,8 @@ __device__ __forceinline__ void tall_density(const CellSpan& c, int ka, int kb, 
     }
 }
 
-// One tall cell, by a team of W threads (in a counted K3 its own thread): an entry
-// in the list of every strip it touches, from which K4 adds its bins in the
+// One tall cell, by a team of W threads (in a counted K3 by its own thread): an
+// entry in the list of every strip it touches, from which K4 adds its bins in the
 // strip's LDS tile.  A strip whose list is full takes the cell's bins in its
 // rows through the side map B instead (marked for K4's fold), and so do all
 // strips of a cell of more than kTallStrips strips or kTallBins bins in a
